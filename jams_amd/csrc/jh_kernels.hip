@@ -420,10 +420,10 @@ __device__ __forceinline__ double cparam(const KParams &p, uint32_t c, int f) {
 __device__ __forceinline__ uint64_t noise_seed(const KParams &p, uint32_t c) {
   return (uint64_t)__double_as_longlong(cparam(p, c, CF_SEED));
 }
-__device__ __forceinline__ uint64_t noise_index_of_ref(const KParams &p, uint32_t c, int64_t ri) {
-  return (uint64_t)ri - (uint64_t)__double_as_longlong(cparam(p, c, CF_ROFF));
+__device__ __forceinline__ uint32_t noise_index_of_ref(const KParams &p, uint32_t c, int64_t ri) {
+  return (uint32_t)((uint64_t)ri - (uint64_t)__double_as_longlong(cparam(p, c, CF_ROFF)));
 }
-__device__ __forceinline__ uint64_t noise_index(const KParams &p, uint32_t c, int64_t i) {
+__device__ __forceinline__ uint32_t noise_index(const KParams &p, uint32_t c, int64_t i) {
   return noise_index_of_ref(p, c, ref_index(p, i));
 }
 
@@ -580,11 +580,10 @@ __device__ __forceinline__ void heun_math(const KParams &p, int64_t i, int64_t r
   if (p.noise == NM_PHILOX && PHASE == 0) {
     double z0, z1, z2, sT;
     if (p.cls) {
-      normals3<false>(noise_seed(p, c), step, noise_index_of_ref(p, c, ri), z0, z1, z2);
+      normals3(noise_seed(p, c), step, noise_index_of_ref(p, c, ri), z0, z1, z2);
       sT = cparam(p, c, CF_SQRTT);
     } else {
-      // one site class: the key schedule stays in scalar registers
-      normals3<true>(p.seed, step, (uint64_t)ri - p.roff, z0, z1, z2);
+      normals3(p.seed, step, (uint32_t)((uint64_t)ri - p.roff), z0, z1, z2);
       sT = p.sqrtT;
     }
     const double sg = cparam(p, c, CF_SIGMA);
@@ -1521,10 +1520,10 @@ __attribute__((amdgpu_waves_per_eu(kMinWaves<PREC, XVk>))) k_rk4(const KParams p
   if (p.noise == NM_PHILOX && stage == 0) {
     double z0, z1, z2, sT;
     if (p.cls) {
-      normals3<false>(noise_seed(p, c), step, noise_index(p, c, i), z0, z1, z2);
+      normals3(noise_seed(p, c), step, noise_index(p, c, i), z0, z1, z2);
       sT = cparam(p, c, CF_SQRTT);
     } else {
-      normals3<true>(p.seed, step, (uint64_t)ref_index(p, i) - p.roff, z0, z1, z2);
+      normals3(p.seed, step, (uint32_t)((uint64_t)ref_index(p, i) - p.roff), z0, z1, z2);
       sT = p.sqrtT;
     }
     const double sg = cparam(p, c, CF_SIGMA);
@@ -1599,7 +1598,7 @@ __global__ void __launch_bounds__(kBlock) k_noise(const KParams p, double *out) 
   if (i >= p.n) return;
   const uint32_t c = p.cls ? (uint32_t)p.cls[i] : 0u;
   double z0, z1, z2;
-  normals3<false>(noise_seed(p, c), p.step, noise_index(p, c, i), z0, z1, z2);
+  normals3(noise_seed(p, c), p.step, noise_index(p, c, i), z0, z1, z2);
   const double sg = cparam(p, c, CF_SIGMA), sT = cparam(p, c, CF_SQRTT);
   out[i] = z0 * sg * sT;
   out[p.n + i] = z1 * sg * sT;
