@@ -511,7 +511,7 @@ void upload_table(jh_ctx *c, const XHost &x, int ntypes, int ntab, int vpt, bool
       const double v = diag ? x.tab[9 * t + 4 * q] : x.tab[9 * t + q];
       t64[(size_t)t * vpt + q] = (c->prec == PR_FP32 && kRoundTables) ? (double)(float)v : v;
     }
-  c->tab64.alloc(t64.size());
+  c->tab64.alloc(t64.size() + t64.size() % 2);  // whole 16-byte words (load_table)
   HIPCHK(hipMemcpy(c->tab64.p, t64.data(), sizeof(double) * t64.size(), hipMemcpyHostToDevice));
 }
 
@@ -1406,7 +1406,7 @@ void prepare_exchange(jh_ctx *c) {
   if (fmt == JH_XFMT_PATTERN || fmt == JH_XFMT_PATTERN_GLOBAL) {
     upload_table(c, x, ntypes, ntab, vpt, diag);
     c->pofs.alloc(pofs.size());
-    c->pat.alloc(pat.size());
+    c->pat.alloc((pat.size() + 3) / 4 * 4);  // whole 16-byte words (load_table)
     HIPCHK(hipMemcpy(c->pofs.p, pofs.data(), sizeof(uint32_t) * pofs.size(), hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(c->pat.p, pat.data(), sizeof(uint32_t) * pat.size(), hipMemcpyHostToDevice));
     c->pat_words = (int)pat.size();
@@ -1441,7 +1441,7 @@ void prepare_exchange(jh_ctx *c) {
           for (uint32_t k = 1; k <= len; ++k)
             up[o + k] = (((int32_t)pat[o + k]) >> tbits) * (int32_t)(kG32 * sizeof(float));
         }
-        c->upat.alloc(up.size());
+        c->upat.alloc((up.size() + 3) / 4 * 4);
         HIPCHK(hipMemcpy(c->upat.p, up.data(), sizeof(int32_t) * up.size(), hipMemcpyHostToDevice));
         c->nuniform = nu;
         c->sseq.alloc(sseq.size());
@@ -1839,11 +1839,12 @@ KParams make_params(jh_ctx *c) {
   // reads 40 % lower in the predictor, 19 % in the corrector, same speed);
   // with long rows the lines run on LINE, and the gathering kernels measured
   // 4 % slower interleaved
-  p.basis_ilv = 0;
-  if (c->order_nb > 1 && !c->xh.empty()) {
+  p.ilv_blocks = 0;
+  if (c->order_nb > 1 && !c->xh.empty() && c->order_cells % c->launch_block() == 0) {
     const XHost &x = c->xh[0];
     const int64_t m = c->n / 2;
-    p.basis_ilv = (x.ptr[m + 1] - x.ptr[m] < kLnAutoMinRow) ? 1 : 0;
+    if (x.ptr[m + 1] - x.ptr[m] < kLnAutoMinRow)
+      p.ilv_blocks = (int)(c->order_cells / c->launch_block());
   }
   return p;
 }

@@ -227,7 +227,9 @@ struct KParams {
   double dt;
   double t;
   int order_nb;         // basis-major period (1: reference order)
-  int basis_ilv;        // gathering step kernels: workgroups alternate basis sites
+  // gathering step kernels: workgroups alternate basis sites, ilv_blocks of
+  // them per site (0: they take the spins in order)
+  int ilv_blocks;
   int ntstore;          // step kernels store their outputs non-temporally
   int64_t order_cells;  // N / order_nb
   double order_rcells;  // 1 / order_cells, rounded

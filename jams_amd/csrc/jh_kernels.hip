@@ -147,12 +147,30 @@ __device__ __forceinline__ void xfield32(const XView &x, const float *__restrict
   h0 = a0; h1 = a1; h2 = a2;
 }
 
-// exchange field of spin i from its row pattern, FP64, reference order
+// f(k, count) over the entries k = 1 .. len of a row in ascending order, in
+// batches of U and then of U/2, ..., 1: the gathers of a batch are issued
+// together, so a row of 6 waits for memory twice with U = 4 and a row of 14
+// four times (entry by entry after the full batches: 3 and 5 times).
+template <int U, class F>
+__device__ __forceinline__ void row_batches(int len, F &&f) {
+  int k = 1;
+  for (; k + U <= len + 1; k += U) f(k, std::integral_constant<int, U>{});
+  if constexpr (U > 1) {
+    const int rest = len + 1 - k;
+    if constexpr (U > 4)
+      if (rest & 4) { f(k, std::integral_constant<int, 4>{}); k += 4; }
+    if constexpr (U > 2)
+      if (rest & 2) { f(k, std::integral_constant<int, 2>{}); k += 2; }
+    if (rest & 1) f(k, std::integral_constant<int, 1>{});
+  }
+}
+
+// exchange field of spin i from its row pattern (at word o), FP64, reference
+// order
 template <int XVk>
 __device__ __forceinline__ void pfield64(const XView &x, const double *__restrict__ src, int64_t n,
-                                         int64_t i, const double *tab, const uint32_t *pat,
-                                         double &h0, double &h1, double &h2) {
-  const uint32_t o = x.pofs[i];
+                                         int64_t i, uint32_t o, const double *tab,
+                                         const uint32_t *pat, double &h0, double &h1, double &h2) {
   const int len = (int)pat[o];
   const uint32_t tmask = (1u << x.tbits) - 1u;
   double a0 = 0.0, a1 = 0.0, a2 = 0.0;
@@ -170,21 +188,30 @@ __device__ __forceinline__ void pfield64(const XView &x, const double *__restric
       a2 = a2 + sx * T[6]; a2 = a2 + sy * T[7]; a2 = a2 + sz * T[8];
     }
   };
-  if (n < ((int64_t)1 << 28)) {
-    // (x, y) pairs and z addressed by 32-bit byte offsets from scalar bases
-    const char *__restrict__ xy = reinterpret_cast<const char *>(src);
-    const char *__restrict__ zs = reinterpret_cast<const char *>(src + 2 * n);
-    const uint32_t ii = (uint32_t)i;
-#pragma unroll kUnrollFor<XVk>
-    for (int k = 1; k <= len; ++k) {
-      const uint32_t w = pat[o + k];
-      const uint32_t j = ii + (uint32_t)(((int32_t)w) >> x.tbits);
-      const double2 v = *reinterpret_cast<const double2 *>(xy + (j << 4));
-      const double sz = *reinterpret_cast<const double *>(zs + (j << 3));
-      accum(w & tmask, v.x, v.y, sz);
-    }
+  // (x, y) pairs and z addressed by 32-bit byte offsets from scalar bases
+  // (a context holds at most 2^31 spins; below 2^28 the offsets fit)
+  const bool small = n < ((int64_t)1 << 28);
+  const char *__restrict__ xy = reinterpret_cast<const char *>(src);
+  const char *__restrict__ zs = reinterpret_cast<const char *>(src + 2 * n);
+  const uint32_t ii = (uint32_t)i;
+  if (small) {
+    row_batches<kUnrollFor<XVk>>(len, [&](int k, auto cnt) {
+      constexpr int C = decltype(cnt)::value;
+      uint32_t w[C];
+      double2 v[C];
+      double z[C];
+#pragma unroll
+      for (int u = 0; u < C; ++u) w[u] = pat[o + k + u];
+#pragma unroll
+      for (int u = 0; u < C; ++u) {
+        const uint32_t j = ii + (uint32_t)(((int32_t)w[u]) >> x.tbits);
+        v[u] = *reinterpret_cast<const double2 *>(xy + (j << 4));
+        z[u] = *reinterpret_cast<const double *>(zs + (j << 3));
+      }
+#pragma unroll
+      for (int u = 0; u < C; ++u) accum(w[u] & tmask, v[u].x, v[u].y, z[u]);
+    });
   } else {
-#pragma unroll kUnrollFor<XVk>
     for (int k = 1; k <= len; ++k) {
       const uint32_t w = pat[o + k];
       const int64_t j = i + (int64_t)(((int32_t)w) >> x.tbits);
@@ -199,31 +226,38 @@ __device__ __forceinline__ void pfield64(const XView &x, const double *__restric
 // the same from FP32 storage with exact FP64 products (see xfield32)
 template <int XVk>
 __device__ __forceinline__ void pfield32(const XView &x, const float *__restrict__ src, int64_t n,
-                                         int64_t i, const double *tab, const uint32_t *pat,
-                                         double &h0, double &h1, double &h2) {
-  const uint32_t o = x.pofs[i];
+                                         int64_t i, uint32_t o, const double *tab,
+                                         const uint32_t *pat, double &h0, double &h1, double &h2) {
   const int len = (int)pat[o];
   const uint32_t tmask = (1u << x.tbits) - 1u;
   double a0 = 0.0, a1 = 0.0, a2 = 0.0;
-#pragma unroll kUnrollFor<XVk>
-  for (int k = 1; k <= len; ++k) {
-    const uint32_t w = pat[o + k];
-    const int64_t j = i + (int64_t)(((int32_t)w) >> x.tbits);
-    const uint32_t t = w & tmask;
-    double sx, sy, sz;
-    load_g32(src, (uint32_t)j, sx, sy, sz);
-    if constexpr (xv_diag(XVk)) {
-      const double *T = tab + __mul24((int)t, 3);
-      a0 = __builtin_fma(sx, T[0], a0);
-      a1 = __builtin_fma(sy, T[1], a1);
-      a2 = __builtin_fma(sz, T[2], a2);
-    } else {
-      const double *T = tab + __mul24((int)t, 9);
-      a0 = __builtin_fma(sx, T[0], a0); a0 = __builtin_fma(sy, T[1], a0); a0 = __builtin_fma(sz, T[2], a0);
-      a1 = __builtin_fma(sx, T[3], a1); a1 = __builtin_fma(sy, T[4], a1); a1 = __builtin_fma(sz, T[5], a1);
-      a2 = __builtin_fma(sx, T[6], a2); a2 = __builtin_fma(sy, T[7], a2); a2 = __builtin_fma(sz, T[8], a2);
+  row_batches<kUnrollFor<XVk>>(len, [&](int k, auto cnt) {
+    constexpr int C = decltype(cnt)::value;
+    uint32_t w[C];
+    double s[C][3];
+#pragma unroll
+    for (int u = 0; u < C; ++u) w[u] = pat[o + k + u];
+#pragma unroll
+    for (int u = 0; u < C; ++u) {
+      const int64_t j = i + (int64_t)(((int32_t)w[u]) >> x.tbits);
+      load_g32(src, (uint32_t)j, s[u][0], s[u][1], s[u][2]);
     }
-  }
+#pragma unroll
+    for (int u = 0; u < C; ++u) {
+      const double sx = s[u][0], sy = s[u][1], sz = s[u][2];
+      if constexpr (xv_diag(XVk)) {
+        const double *T = tab + __mul24((int)(w[u] & tmask), 3);
+        a0 = __builtin_fma(sx, T[0], a0);
+        a1 = __builtin_fma(sy, T[1], a1);
+        a2 = __builtin_fma(sz, T[2], a2);
+      } else {
+        const double *T = tab + __mul24((int)(w[u] & tmask), 9);
+        a0 = __builtin_fma(sx, T[0], a0); a0 = __builtin_fma(sy, T[1], a0); a0 = __builtin_fma(sz, T[2], a0);
+        a1 = __builtin_fma(sx, T[3], a1); a1 = __builtin_fma(sy, T[4], a1); a1 = __builtin_fma(sz, T[5], a1);
+        a2 = __builtin_fma(sx, T[6], a2); a2 = __builtin_fma(sy, T[7], a2); a2 = __builtin_fma(sz, T[8], a2);
+      }
+    }
+  });
   h0 = a0; h1 = a1; h2 = a2;
 }
 
@@ -235,40 +269,49 @@ __device__ __forceinline__ void pfield32(const XView &x, const float *__restrict
 // gpat: the (offset, tensor id) words for the non-uniform slices (global).
 template <int XVk>
 __device__ __forceinline__ void ufield32(const XView &x, const float *__restrict__ src, int64_t n,
-                                         int64_t i, const double *tab, const int32_t *upat,
-                                         const uint32_t *gpat, double &h0, double &h1,
-                                         double &h2) {
+                                         int64_t i, uint32_t o, const double *tab,
+                                         const int32_t *upat, const uint32_t *gpat, double &h0,
+                                         double &h1, double &h2) {
   const int sl = __builtin_amdgcn_readfirstlane((int)(i >> 6));
   const int2 info = x.sseq[sl];
   const int soff = __builtin_amdgcn_readfirstlane(info.x);
   if (soff < 0) {
-    pfield32<XVk>(x, src, n, i, tab, gpat, h0, h1, h2);
+    pfield32<XVk>(x, src, n, i, o, tab, gpat, h0, h1, h2);
     return;
   }
   const int len = __builtin_amdgcn_readfirstlane(info.y);
   const double *__restrict__ T = x.seqtab + soff;
-  const uint32_t o = x.pofs[i];
   // byte offset of this spin in the gather copy (the copy is < 2 GiB)
   const uint32_t ib = (uint32_t)i * (uint32_t)(kG32 * sizeof(float));
   const char *__restrict__ base = reinterpret_cast<const char *>(src);
   double a0 = 0.0, a1 = 0.0, a2 = 0.0;
-#pragma unroll kUnrollFor<XVk>
-  for (int k = 0; k < len; ++k) {
-    const uint32_t jb = ib + (uint32_t)upat[o + 1 + k];
-    const float *q = reinterpret_cast<const float *>(base + jb);
-    const double sx = q[0], sy = q[1], sz = q[2];
-    if constexpr (xv_diag(XVk)) {
-      const double *Tk = T + 3 * k;
-      a0 = __builtin_fma(sx, Tk[0], a0);
-      a1 = __builtin_fma(sy, Tk[1], a1);
-      a2 = __builtin_fma(sz, Tk[2], a2);
-    } else {
-      const double *Tk = T + 9 * k;
-      a0 = __builtin_fma(sx, Tk[0], a0); a0 = __builtin_fma(sy, Tk[1], a0); a0 = __builtin_fma(sz, Tk[2], a0);
-      a1 = __builtin_fma(sx, Tk[3], a1); a1 = __builtin_fma(sy, Tk[4], a1); a1 = __builtin_fma(sz, Tk[5], a1);
-      a2 = __builtin_fma(sx, Tk[6], a2); a2 = __builtin_fma(sy, Tk[7], a2); a2 = __builtin_fma(sz, Tk[8], a2);
+  row_batches<kUnrollFor<XVk>>(len, [&](int k, auto cnt) {
+    constexpr int C = decltype(cnt)::value;
+    uint32_t jb[C];
+    double s[C][3];
+#pragma unroll
+    for (int u = 0; u < C; ++u) jb[u] = ib + (uint32_t)upat[o + k + u];
+#pragma unroll
+    for (int u = 0; u < C; ++u) {
+      const float *q = reinterpret_cast<const float *>(base + jb[u]);
+      s[u][0] = q[0]; s[u][1] = q[1]; s[u][2] = q[2];
     }
-  }
+#pragma unroll
+    for (int u = 0; u < C; ++u) {
+      const double sx = s[u][0], sy = s[u][1], sz = s[u][2];
+      if constexpr (xv_diag(XVk)) {
+        const double *Tk = T + 3 * (k - 1 + u);
+        a0 = __builtin_fma(sx, Tk[0], a0);
+        a1 = __builtin_fma(sy, Tk[1], a1);
+        a2 = __builtin_fma(sz, Tk[2], a2);
+      } else {
+        const double *Tk = T + 9 * (k - 1 + u);
+        a0 = __builtin_fma(sx, Tk[0], a0); a0 = __builtin_fma(sy, Tk[1], a0); a0 = __builtin_fma(sz, Tk[2], a0);
+        a1 = __builtin_fma(sx, Tk[3], a1); a1 = __builtin_fma(sy, Tk[4], a1); a1 = __builtin_fma(sz, Tk[5], a1);
+        a2 = __builtin_fma(sx, Tk[6], a2); a2 = __builtin_fma(sy, Tk[7], a2); a2 = __builtin_fma(sz, Tk[8], a2);
+      }
+    }
+  });
   h0 = a0; h1 = a1; h2 = a2;
 }
 
@@ -287,21 +330,21 @@ __device__ __forceinline__ void dmi_add(const double *__restrict__ D, float bx, 
 // plus D x (s1 - s2) per pair in FP64 (QDMI).  Other slices take ufield32.
 template <int XVk>
 __device__ __forceinline__ void pairfield32(const XView &x, const float *__restrict__ src,
-                                            int64_t n, int64_t i, const double *tab,
+                                            int64_t n, int64_t i, uint32_t row, const double *tab,
                                             const int32_t *upat, const uint32_t *gpat,
                                             double &h0, double &h1, double &h2) {
   const int sl = __builtin_amdgcn_readfirstlane((int)(i >> 6));
   const int2 info = x.spair[sl];
   const int g0 = __builtin_amdgcn_readfirstlane(info.x);
   if (g0 < 0) {
-    ufield32<XVk>(x, src, n, i, tab, upat, gpat, h0, h1, h2);
+    ufield32<XVk>(x, src, n, i, row, tab, upat, gpat, h0, h1, h2);
     return;
   }
   const int cnt = __builtin_amdgcn_readfirstlane(info.y);
   const int n2 = cnt & 0xFFFF, n1 = cnt >> 16;
   const int4 *__restrict__ G = x.pgrp + g0;
   const double *__restrict__ V = x.pval + (size_t)8 * g0;
-  const uint32_t o = x.pofs[i] + 1;
+  const uint32_t o = row + 1;
   // byte offset of this spin in the gather copy (the copy is < 2 GiB)
   const uint32_t ib = (uint32_t)i * (uint32_t)(kG32 * sizeof(float));
   const char *__restrict__ base = reinterpret_cast<const char *>(src);
@@ -355,35 +398,52 @@ __host__ __device__ inline size_t table_bytes(int prec, int xv, int ntab) {
   return (b + 15) & ~(size_t)15;
 }
 
-// Copy `words` 32-bit words global -> LDS (both 16-byte aligned) with
-// 16-byte loads: every workgroup stages the tables, so their load count
-// matters (the five-shell bcc pattern table is 7552 words).
-__device__ __forceinline__ void copy_words(uint32_t *dst, const uint32_t *__restrict__ src,
-                                           int words) {
-  const int w4 = words >> 2;
-  uint4 *d4 = reinterpret_cast<uint4 *>(dst);
-  const uint4 *s4 = reinterpret_cast<const uint4 *>(src);
-  for (int q = threadIdx.x; q < w4; q += blockDim.x) d4[q] = s4[q];
-  for (int q = (w4 << 2) + (int)threadIdx.x; q < words; q += blockDim.x) dst[q] = src[q];
-}
-
+// Stage the tensor table and the pattern words in LDS (both tables are padded
+// to 16 bytes on the device).  Every workgroup does this before it can start,
+// so the copy is one pass over both with 16-byte loads, kStage of a thread's
+// loads in flight together: one wait for memory where the tables fit in
+// kStage * blockDim words of 16 bytes (all that fit in 48 KB do at 512
+// threads).
+constexpr int kStage = 6;
+typedef uint32_t u32v4 __attribute__((ext_vector_type(4)));
 template <int PREC, int XVk>
 __device__ __forceinline__ void load_table(const XView &x, unsigned char *lds) {
   if constexpr (xv_typed(XVk)) {
-    const int cnt = x.ntab * (xv_diag(XVk) ? 3 : 9);
-    copy_words(reinterpret_cast<uint32_t *>(lds), reinterpret_cast<const uint32_t *>(x.tab64),
-               2 * cnt);
+    const int nt = (int)(table_bytes(PREC, XVk, x.ntab) >> 4);
+    const int np = xv_pattern_lds(XVk) ? (x.pat_words + 3) >> 2 : 0;
+    const u32v4 *st = reinterpret_cast<const u32v4 *>(x.tab64);
+    const u32v4 *sp = reinterpret_cast<const u32v4 *>(
+        xv_uniform(XVk) ? reinterpret_cast<const uint32_t *>(x.upat) : x.pat);
+    u32v4 *d = reinterpret_cast<u32v4 *>(lds);
+    const int total = nt + np, step = (int)blockDim.x;
+    for (int q0 = 0; q0 < total; q0 += kStage * step) {
+      u32v4 v[kStage];
+#pragma unroll
+      for (int u = 0; u < kStage; ++u) {
+        if (q0 + u * step >= total) break;  // the same in every lane
+        const int q = min(q0 + u * step + (int)threadIdx.x, total - 1);
+        v[u] = q < nt ? st[q] : sp[q - nt];
+      }
+#pragma unroll
+      for (int u = 0; u < kStage; ++u) {
+        const int q = q0 + u * step + (int)threadIdx.x;
+        if (q < total) d[q] = v[u];
+      }
+    }
   }
-  if constexpr (xv_pattern_lds(XVk)) {
-    uint32_t *p = reinterpret_cast<uint32_t *>(lds + table_bytes(PREC, XVk, x.ntab));
-    const uint32_t *from = xv_uniform(XVk) ? reinterpret_cast<const uint32_t *>(x.upat) : x.pat;
-    copy_words(p, from, x.pat_words);
-  }
+}
+
+// the word of spin i's row pattern (pattern formats); loaded before the
+// tables are staged so that the two waits overlap
+template <int XVk>
+__device__ __forceinline__ uint32_t row_word(const XView &x, int64_t i) {
+  if constexpr (xv_pattern(XVk)) return x.pofs[i];
+  else return 0u;
 }
 
 template <int PREC, int XVk>
 __device__ __forceinline__ void exchange_at(const KParams &p, const double *src64,
-                                            const float *src32, int64_t i,
+                                            const float *src32, int64_t i, uint32_t row,
                                             const unsigned char *lds, double &f0, double &f1,
                                             double &f2) {
   if constexpr (XVk == XV_NONE) {
@@ -395,15 +455,15 @@ __device__ __forceinline__ void exchange_at(const KParams &p, const double *src6
     else
       pat = p.x.pat;
     if constexpr (PREC == PR_FP64)
-      pfield64<XVk>(p.x, src64, p.n, i, reinterpret_cast<const double *>(lds), pat, f0, f1, f2);
+      pfield64<XVk>(p.x, src64, p.n, i, row, reinterpret_cast<const double *>(lds), pat, f0, f1, f2);
     else if constexpr (xv_pair(XVk))
-      pairfield32<XVk>(p.x, src32, p.n, i, reinterpret_cast<const double *>(lds),
+      pairfield32<XVk>(p.x, src32, p.n, i, row, reinterpret_cast<const double *>(lds),
                        reinterpret_cast<const int32_t *>(pat), p.x.pat, f0, f1, f2);
     else if constexpr (xv_uniform(XVk))
-      ufield32<XVk>(p.x, src32, p.n, i, reinterpret_cast<const double *>(lds),
+      ufield32<XVk>(p.x, src32, p.n, i, row, reinterpret_cast<const double *>(lds),
                     reinterpret_cast<const int32_t *>(pat), p.x.pat, f0, f1, f2);
     else
-      pfield32<XVk>(p.x, src32, p.n, i, reinterpret_cast<const double *>(lds), pat, f0, f1, f2);
+      pfield32<XVk>(p.x, src32, p.n, i, row, reinterpret_cast<const double *>(lds), pat, f0, f1, f2);
   } else if constexpr (PREC == PR_FP64) {
     xfield64<XVk>(p.x, src64, p.n, i, reinterpret_cast<const double *>(lds), f0, f1, f2);
   } else {
@@ -489,12 +549,12 @@ __device__ __forceinline__ void sum_terms(const KParams &p, uint32_t c, int64_t 
 
 template <int PREC, int XVk, bool GEN>
 __device__ __forceinline__ void total_field(const KParams &p, const double *src64,
-                                            const float *src32, int64_t i, uint32_t c,
+                                            const float *src32, int64_t i, uint32_t row, uint32_t c,
                                             const unsigned char *lds, double s0, double s1,
                                             double s2, double t, double &h0, double &h1,
                                             double &h2) {
   double x0, x1, x2;
-  exchange_at<PREC, XVk>(p, src64, src32, i, lds, x0, x1, x2);
+  exchange_at<PREC, XVk>(p, src64, src32, i, row, lds, x0, x1, x2);
   sum_terms<GEN>(p, c, i, s0, s1, s2, t, x0, x1, x2, h0, h1, h2);
 }
 
@@ -686,14 +746,15 @@ constexpr int kMinWaves = (PREC == PR_FP32 && xv_uniform(XVk)) ? JH_UNIFORM_WAVE
                           : xv_diag(XVk) ? JH_DIAG_WAVES : JH_WAVES_PER_EU;
 
 // The spin block a gathering step kernel's workgroup takes for its XCD-
-// ordered block number blk.  With basis_ilv the workgroups alternate between
+// ordered block number blk.  With ilv_blocks the workgroups alternate between
 // the basis sites' index ranges, so the workgroups of one XCD hold the same
 // cells of every basis site and the other sites' spins their rows gather stay
 // in that XCD's L2.
 __device__ __forceinline__ int64_t step_block(const KParams &p, int64_t blk) {
-  if (p.basis_ilv && !p.rowlist && p.order_nb > 1 && p.order_cells % blockDim.x == 0) {
-    const int64_t per = p.order_cells / blockDim.x;
-    blk = (blk % p.order_nb) * per + blk / p.order_nb;
+  if (p.ilv_blocks > 0 && !p.rowlist) {
+    // 32-bit: the 64-bit divisions were 600 scalar instructions per wave
+    const uint32_t b = (uint32_t)blk, q = b / (uint32_t)p.order_nb;
+    return (int64_t)(b - q * (uint32_t)p.order_nb) * p.ilv_blocks + q;
   }
   return blk;
 }
@@ -712,20 +773,33 @@ __device__ __forceinline__ int64_t step_block(const KParams &p, int64_t blk) {
 //   CM_ONE:   no class table: every spin has class 0, known at compile time.
 enum { CM_LANE = 0, CM_SPLIT = 1, CM_ONE = 2 };
 
+// What a gathering phase reads of its spin before its field: the row word,
+// the class and the spin the field is evaluated at.
+struct GatherPre {
+  uint32_t row, c;
+  double s0, s1, s2;
+  OwnState own;
+};
+template <int PREC, int XVk, int PHASE, int CM>
+__device__ __forceinline__ void gather_pre(const KParams &p, int64_t i, GatherPre &g) {
+  g.row = row_word<XVk>(p.x, i);
+  g.c = CM == CM_ONE ? 0u : p.cls ? (uint32_t)p.cls[i] : 0u;
+  phase_spin<PREC, PHASE>(p, i, g.s0, g.s1, g.s2, g.own);
+}
+
 // One Heun phase of spin i with the gathering exchange formats: the field at
 // the phase's spins and the phase's update and stores.
 template <int PREC, int XVk, int PHASE, bool GEN, int CM = CM_LANE>
-__device__ __forceinline__ void heun_gather_spin(const KParams &p, int64_t i,
+__device__ __forceinline__ void heun_gather_spin(const KParams &p, int64_t i, const GatherPre &g,
                                                  const unsigned char *lds) {
-  const uint32_t c = CM == CM_ONE ? 0u : p.cls ? (uint32_t)p.cls[i] : 0u;
+  const uint32_t c = g.c;
   const uint64_t step = launch_step(p);
   const double t0 = launch_time(p, step);
-  double s0, s1, s2;
-  OwnState own;
-  phase_spin<PREC, PHASE>(p, i, s0, s1, s2, own);
+  const double s0 = g.s0, s1 = g.s1, s2 = g.s2;
+  const OwnState &own = g.own;
   const double t = PHASE == 0 ? t0 : t0 + p.dt;
   double x0, x1, x2;
-  exchange_at<PREC, XVk>(p, PHASE == 0 ? p.s : p.sp, p.g32, i, lds, x0, x1, x2);
+  exchange_at<PREC, XVk>(p, PHASE == 0 ? p.s : p.sp, p.g32, i, g.row, lds, x0, x1, x2);
   if constexpr (CM == CM_SPLIT) {
     const uint32_t c0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)c);
     if (__builtin_amdgcn_ballot_w64(c != c0) == 0)
@@ -741,16 +815,17 @@ template <int PREC, int XVk, int PHASE, bool GEN, int CM>
 __global__ void __launch_bounds__(kMaxBlock)
 __attribute__((amdgpu_waves_per_eu(kMinWaves<PREC, XVk>))) k_heun(const KParams p) {
   extern __shared__ __align__(16) unsigned char lds[];
+  int64_t i = step_block(p, xcd_block(blockIdx.x, gridDim.x)) * blockDim.x + threadIdx.x;
+  const bool live = i < (p.rowlist ? p.nrowlist : p.n);
+  GatherPre g;
+  if (live) {
+    if (p.rowlist) i = p.rowlist[i];
+    gather_pre<PREC, XVk, PHASE, CM>(p, i, g);
+  }
   load_table<PREC, XVk>(p.x, lds);
   if constexpr (xv_typed(XVk)) __syncthreads();
-  int64_t i = step_block(p, xcd_block(blockIdx.x, gridDim.x)) * blockDim.x + threadIdx.x;
-  if (p.rowlist) {
-    if (i >= p.nrowlist) return;
-    i = p.rowlist[i];
-  } else if (i >= p.n) {
-    return;
-  }
-  heun_gather_spin<PREC, XVk, PHASE, GEN, CM>(p, i, lds);
+  if (!live) return;
+  heun_gather_spin<PREC, XVk, PHASE, GEN, CM>(p, i, g, lds);
 }
 
 // Grid barrier of the persistent step kernel over sync = {arrived count,
@@ -811,7 +886,11 @@ k_heun_step(const KParams p, unsigned *sync, unsigned limit) {
   const int64_t nv = (p.n + blockDim.x - 1) / blockDim.x;
   for (int64_t v = blockIdx.x; v < nv; v += gridDim.x) {
     const int64_t i = step_block(p, xcd_block(v, nv)) * blockDim.x + threadIdx.x;
-    if (i < p.n) heun_gather_spin<PREC, XVk, 0, GEN>(p, i, lds);
+    if (i < p.n) {
+      GatherPre g;
+      gather_pre<PREC, XVk, 0, CM_LANE>(p, i, g);
+      heun_gather_spin<PREC, XVk, 0, GEN>(p, i, g, lds);
+    }
   }
   if (!grid_barrier(sync, limit)) return;
   KParams q = p;
@@ -819,7 +898,11 @@ k_heun_step(const KParams p, unsigned *sync, unsigned limit) {
   q.w32 = const_cast<float *>(p.g32);
   for (int64_t v = blockIdx.x; v < nv; v += gridDim.x) {
     const int64_t i = step_block(q, xcd_block(v, nv)) * blockDim.x + threadIdx.x;
-    if (i < q.n) heun_gather_spin<PREC, XVk, 1, GEN>(q, i, lds);
+    if (i < q.n) {
+      GatherPre g;
+      gather_pre<PREC, XVk, 1, CM_LANE>(q, i, g);
+      heun_gather_spin<PREC, XVk, 1, GEN>(q, i, g, lds);
+    }
   }
 }
 
@@ -1363,21 +1446,19 @@ __attribute__((amdgpu_waves_per_eu(kLnWaves<PHASE>))) k_heun_ln(const KParams p,
     if constexpr (PREC == PR_FP64) {
       extern __shared__ __align__(16) unsigned char lds[];
       constexpr int XG = DIAG ? XV_GDIAG : XV_GFULL;
+      const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+      const bool live = j < ln.nrows;
+      constexpr int CM = ONE ? CM_ONE : CM_LANE;
+      int64_t i = 0;
+      GatherPre g;
+      if (live) {
+        i = ln.rows[j];
+        gather_pre<PREC, XG, PHASE, CM>(p, i, g);
+      }
       load_table<PREC, XG>(p.x, lds);
       __syncthreads();
-      const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-      if (j >= ln.nrows) return;
-      const int64_t i = ln.rows[j];
-      const uint32_t c = ONE ? 0u : p.cls ? (uint32_t)p.cls[i] : 0u;
-      const uint64_t step = launch_step(p);
-      const double t0 = launch_time(p, step);
-      double s0, s1, s2;
-      OwnState own;
-      phase_spin<PREC, PHASE>(p, i, s0, s1, s2, own);
-      const double t = PHASE == 0 ? t0 : t0 + p.dt;
-      double x0, x1, x2;
-      exchange_at<PREC, XG>(p, PHASE == 0 ? p.s : p.sp, p.g32, i, lds, x0, x1, x2);
-      heun_spin<PREC, PHASE, GEN>(p, i, c, step, t, s0, s1, s2, x0, x1, x2, own);
+      if (!live) return;
+      heun_gather_spin<PREC, XG, PHASE, GEN, CM>(p, i, g, lds);
     }
     return;
   }
@@ -1388,14 +1469,17 @@ __attribute__((amdgpu_waves_per_eu(kLnWaves<PHASE>))) k_heun_ln(const KParams p,
   // other, run side by side on one XCD, and the lines in flight on an XCD
   // stay within a few x of each other in one band, so their neighbour lines
   // stay in its L2
-  const int64_t q = blk * (int64_t)(blockDim.x >> 6) + wave;
+  // (32-bit: fewer than 2^31 cells; 64-bit divisions take 130 scalar
+  // instructions each)
+  const uint32_t q = (uint32_t)blk * (blockDim.x >> 6) + (uint32_t)wave;
   const int lane = (int)(threadIdx.x & 63);
-  const int b = (int)(q % ln.nb);
-  int64_t r = q / ln.nb;
-  const int yin = (int)(r % ln.ty);
-  r /= ln.ty;
-  const int xw = (int)(r % ln.lx);
-  const int yw = (int)(r / ln.lx) * ln.ty + yin;
+  const uint32_t qb = q / (uint32_t)ln.nb;
+  const int b = (int)(q - qb * (uint32_t)ln.nb);
+  const uint32_t qy = qb / (uint32_t)ln.ty;
+  const int yin = (int)(qb - qy * (uint32_t)ln.ty);
+  const uint32_t qx = qy / (uint32_t)ln.lx;
+  const int xw = (int)(qy - qx * (uint32_t)ln.lx);
+  const int yw = (int)qx * ln.ty + yin;
   const int64_t line = ((int64_t)b * ln.lx + xw) * ln.ly + yw;
   const int64_t i0 = line * ln.lz + (int64_t)P * lane;
   const int64_t n = p.n;
@@ -1497,24 +1581,29 @@ template <int PREC, int XVk, bool GEN, bool ONE>
 __global__ void __launch_bounds__(kMaxBlock)
 __attribute__((amdgpu_waves_per_eu(kMinWaves<PREC, XVk>))) k_rk4(const KParams p) {
   extern __shared__ __align__(16) unsigned char lds[];
-  load_table<PREC, XVk>(p.x, lds);
-  if constexpr (xv_typed(XVk)) __syncthreads();
   const int64_t blk = xcd_block(blockIdx.x, gridDim.x);
   const int64_t i = blk * blockDim.x + threadIdx.x;
-  if (i >= p.n) return;
+  const bool live = i < p.n;
   const int64_t n = p.n;
-  const uint32_t c = ONE ? 0u : p.cls ? (uint32_t)p.cls[i] : 0u;
   const int stage = p.stage;
+  const double *src = stage == 0 ? p.s : p.sp;
+  uint32_t c = 0, row = 0;
+  double y0 = 0.0, y1 = 0.0, y2 = 0.0;
+  if (live) {
+    row = row_word<XVk>(p.x, i);
+    if (!ONE && p.cls) c = (uint32_t)p.cls[i];
+    load_spin(src, n, i, y0, y1, y2);
+  }
+  load_table<PREC, XVk>(p.x, lds);
+  if constexpr (xv_typed(XVk)) __syncthreads();
+  if (!live) return;
   const uint64_t step = p.dstep ? *p.dstep + p.step : p.step;
   const double t0 = p.dstep ? (double)step * p.dt : p.t;
   const double half = 0.5 * p.dt;
   const double t = stage == 0 ? t0 : stage == 3 ? t0 + p.dt : t0 + half;
 
-  const double *src = stage == 0 ? p.s : p.sp;
-  double y0, y1, y2;
-  load_spin(src, n, i, y0, y1, y2);
   double h0, h1, h2;
-  total_field<PREC, XVk, GEN>(p, src, p.g32, i, c, lds, y0, y1, y2, t, h0, h1, h2);
+  total_field<PREC, XVk, GEN>(p, src, p.g32, i, row, c, lds, y0, y1, y2, t, h0, h1, h2);
 
   double w0 = 0.0, w1 = 0.0, w2 = 0.0;
   if (p.noise == NM_PHILOX && stage == 0) {
@@ -1583,9 +1672,9 @@ __global__ void __launch_bounds__(kBlock) k_field(const KParams p, int term, dou
   load_spin(p.s, n, i, s0, s1, s2);
   double h0, h1, h2;
   if (term < 0) {
-    total_field<PREC, XVk, true>(p, p.s, p.g32, i, c, lds, s0, s1, s2, p.t, h0, h1, h2);
+    total_field<PREC, XVk, true>(p, p.s, p.g32, i, row_word<XVk>(p.x, i), c, lds, s0, s1, s2, p.t, h0, h1, h2);
   } else if (p.kind[term] == TK_EXCHANGE) {
-    exchange_at<PREC, XVk>(p, p.s, p.g32, i, lds, h0, h1, h2);
+    exchange_at<PREC, XVk>(p, p.s, p.g32, i, row_word<XVk>(p.x, i), lds, h0, h1, h2);
   } else {
     local_term<true>(p, p.kind[term], c, i, s0, s1, s2, p.t, h0, h1, h2);
   }
@@ -1705,7 +1794,7 @@ __global__ void k_set_step(uint64_t *step, uint64_t value) {
 
 static size_t table_lds(const KParams &p, int prec, int xv) {
   size_t b = table_bytes(prec, xv, p.x.ntab);
-  if (xv_pattern_lds(xv)) b += (size_t)p.x.pat_words * 4;
+  if (xv_pattern_lds(xv)) b += ((size_t)p.x.pat_words * 4 + 15) & ~(size_t)15;
   return b;
 }
 
