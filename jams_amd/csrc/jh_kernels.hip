@@ -1784,6 +1784,43 @@ __global__ void __launch_bounds__(kBlock) k_reduce_replicas(const KParams p, con
   if (threadIdx.x < 4) out[(int64_t)r * 4 + threadIdx.x] = red[threadIdx.x][0];
 }
 
+// Host layout (N x 3, reference order) <-> device layout of a vector array: a
+// workgroup moves kBlock spins, consecutive in the reference order, through
+// LDS so that the host side is read and written in whole consecutive words
+// (the destination may be mapped host memory).
+template <bool SPIN, bool TO_HOST>
+__global__ void __launch_bounds__(kBlock) k_vec_layout(const double *in, double *out, int64_t n,
+                                                       int order_nb, int64_t order_cells) {
+  __shared__ double v[3 * kBlock];
+  const int64_t i0 = (int64_t)blockIdx.x * kBlock;
+  const int m = (int)min((int64_t)kBlock, n - i0), tid = (int)threadIdx.x;
+  if constexpr (!TO_HOST) {
+    for (int e = tid; e < 3 * m; e += kBlock) v[e] = in[3 * i0 + e];
+    __syncthreads();
+  }
+  if (tid < m) {
+    const uint32_t i = (uint32_t)(i0 + tid);
+    const uint32_t cell = i / (uint32_t)order_nb;
+    const int64_t d = order_nb == 1 ? (int64_t)i
+                                    : (int64_t)(i - cell * (uint32_t)order_nb) * order_cells + cell;
+    if constexpr (TO_HOST) {
+      if constexpr (SPIN) {
+        load_spin(in, n, d, v[3 * tid], v[3 * tid + 1], v[3 * tid + 2]);
+      } else {
+        for (int c = 0; c < 3; ++c) v[3 * tid + c] = in[c * n + d];
+      }
+    } else if constexpr (SPIN) {
+      store_spin(out, n, d, v[3 * tid], v[3 * tid + 1], v[3 * tid + 2]);
+    } else {
+      for (int c = 0; c < 3; ++c) out[c * n + d] = v[3 * tid + c];
+    }
+  }
+  if constexpr (TO_HOST) {
+    __syncthreads();
+    for (int e = tid; e < 3 * m; e += kBlock) out[3 * i0 + e] = v[e];
+  }
+}
+
 // One thread sets the device step counter of a graph replay.
 __global__ void k_set_step(uint64_t *step, uint64_t value) {
   if (blockIdx.x == 0 && threadIdx.x == 0) *step = value;
@@ -2118,6 +2155,15 @@ hipError_t launch_field(const KParams &p, int prec, int xv, int term, double *ou
                         hipStream_t st) {
   return prec == PR_FP64 ? launch_field_p<PR_FP64>(p, xv, term, out, st)
                          : launch_field_p<PR_FP32>(p, xv, term, out, st);
+}
+
+hipError_t launch_vec_layout(const double *in, double *out, int64_t n, int order_nb,
+                             int64_t order_cells, bool spin, bool to_host, hipStream_t st) {
+  const auto fn = spin ? (to_host ? k_vec_layout<true, true> : k_vec_layout<true, false>)
+                       : (to_host ? k_vec_layout<false, true> : k_vec_layout<false, false>);
+  const int64_t nb = (n + kBlock - 1) / kBlock;
+  hipLaunchKernelGGL(fn, dim3((unsigned)nb), dim3(kBlock), 0, st, in, out, n, order_nb, order_cells);
+  return hipGetLastError();
 }
 
 hipError_t launch_noise(const KParams &p, double *out, hipStream_t st) {

@@ -30,6 +30,10 @@ hipError_t launch_reduce_replicas(const KParams &p, const int64_t *off, int nrep
 hipError_t launch_set_step(uint64_t *step, uint64_t value, hipStream_t st);
 hipError_t launch_field(const KParams &p, int prec, int xv, int term, double *out,
                         hipStream_t st);
+// a vector array between the host layout (N x 3, reference order) and the
+// device layout (a spin array or SoA, device order)
+hipError_t launch_vec_layout(const double *in, double *out, int64_t n, int order_nb,
+                             int64_t order_cells, bool spin, bool to_host, hipStream_t st);
 hipError_t launch_noise(const KParams &p, double *out, hipStream_t st);
 hipError_t launch_to_f32(const double *a, float *b, int64_t m, hipStream_t st);
 hipError_t launch_reduce(const KParams &p, int mode, const double *h, double *partial,
