@@ -84,6 +84,14 @@ constexpr int64_t kLnAutoMinRow = 24;           // neighbours per row from which
 // typically about a second, against a phase of under a millisecond for a few
 // million spins
 constexpr unsigned kStepPollLimit = 1u << 20;
+// steps of one launch of k_heun_many (a few ms at most)
+constexpr int kManyStepsMax = 1024;
+// vector operations per step (spins x operations per spin) up to which
+// k_heun_many, on one compute unit, is faster than two launches on all of
+// them: sc 10^3 thermal (0.78 M) 7.0 against 11.8 us, bcc 8^3 x 2 two shells
+// thermal (0.96 M) 9.7 against 13.9; at 1.6 M (sc 11^3 to 12^3, two spins per
+// thread) 10 to 13 against 11 to 12
+constexpr double kManyOps = 1.2e6;
 // spins from which the step kernels store their outputs non-temporally
 constexpr int64_t kNtStoreMin = (int64_t)1 << 21;
 constexpr int kLnBand = JH_LN_BAND;             // y rows per band of the LINE wave order
@@ -2062,8 +2070,34 @@ void build_graph(jh_ctx *c) {
   HIPCHK(hipGraphInstantiate(&c->gexec, c->graph, nullptr, nullptr, 0));
 }
 
+// Whether the context's steps run as many steps per launch of one workgroup
+// (k_heun_many).
+bool many_steps(const jh_ctx *c) {
+  if (c->integrator != JH_INTEGRATOR_HEUN || c->step_launch != JH_STEP_LAUNCH_TWO || c->block ||
+      c->st_on || c->ln_on || c->n > kManySpins || c->nclass != 1 || c->has_ac ||
+      c->ani_power != 2 || dipole_term(c) >= 0 || !heun_many_variant(c->prec, c->xv))
+    return false;
+  const double nbrs = c->xh.empty() ? 0.0 : (double)c->xh[0].ptr[c->n] / (double)c->n;
+  const bool hot = c->noise_mode == NM_PHILOX;
+  const double ops = 2.0 * (nbrs * 10.0 + 200.0) + (hot ? 260.0 : 0.0);
+  return (double)c->n * ops < kManyOps;
+}
+
 void do_steps(jh_ctx *c, int64_t nsteps) {
   int64_t done = 0;
+  if (many_steps(c)) {
+    KParams p = make_params(c);
+    p.w32 = c->s32.p;
+    while (done < nsteps) {
+      const int k = (int)std::min<int64_t>(nsteps - done, kManyStepsMax);
+      p.step = (uint64_t)c->iteration;
+      HIPCHK(launch_heun_many(p, c->prec, c->xv, k, c->stream));
+      done += k;
+      c->iteration += k;
+      c->time = (double)c->iteration * c->dt;
+    }
+    return;
+  }
   if (c->graph_steps > 0 && nsteps >= c->graph_steps) {
     if (!c->gexec) build_graph(c);
     for (; done + c->graph_steps <= nsteps; done += c->graph_steps) {

@@ -41,6 +41,8 @@ namespace jh {
 
 constexpr int kBlock = 256;          // threads per workgroup of the helper kernels
 constexpr int kMaxBlock = 512;       // largest step-kernel workgroup (autotuned)
+constexpr int kManySpins = 1024;     // spins of the small systems' many-step launch,
+                                     // one per thread (two held too many registers)
 constexpr int kSlice = 64;           // spins per ELL slice (one wavefront)
 constexpr uint32_t kPad = 0xFFFFFFFFu;
 #ifndef JH_G32

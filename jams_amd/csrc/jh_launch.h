@@ -15,6 +15,10 @@ hipError_t launch_heun(const KParams &p, int prec, int xv, int phase, int bs, hi
 // a workgroup gives the barrier up and sets sync[2]
 hipError_t launch_heun_step(const KParams &p, int prec, int xv, int bs, int cus, unsigned *sync,
                             unsigned limit, hipStream_t st);
+// nsteps whole Heun steps of a small system in one workgroup (steps p.step,
+// p.step + 1, ...; p.w32: the FP32 copy of s); one site class, no dipole term
+bool heun_many_variant(int prec, int xv);
+hipError_t launch_heun_many(const KParams &p, int prec, int xv, int nsteps, hipStream_t st);
 // one Heun phase over the STENCIL layout v, full or diagonal tensors
 hipError_t launch_heun_st(const KParams &p, const StView &v, int prec, bool diag, int phase,
                           hipStream_t st);

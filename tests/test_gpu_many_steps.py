@@ -1,0 +1,73 @@
+"""Small systems run many Heun steps in one launch of one workgroup: bit for
+bit the two-launch kernels (which an explicit workgroup size selects), at the
+smallest sizes, at wave edges and at the largest, with and without noise, in
+both precision forms, across calls of any length."""
+import numpy as np
+import pytest
+
+from jams_amd import configs
+from jams_amd.host import Simulation
+from oracle import pyoracle as po
+from tests import systems as S
+
+pytestmark = pytest.mark.gpu
+
+
+def run(text, block, calls):
+    sim = Simulation(text, device=0, output_dir="/tmp")
+    e = sim.engine()
+    e.set_block_size(block)
+    out = []
+    for n in calls:
+        e.step(n)
+        out.append((e.get_spins(), e.iteration(), e.magnetisation()))
+    sim.close()
+    return out
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32-field"])
+@pytest.mark.parametrize("L,open_ends,T", [
+    ((2, 1, 1), True, 5.0), ((3, 3, 7), False, 10.0), ((4, 4, 4), False, 0.0), ((5, 13, 1), True, 300.0),
+    ((8, 8, 8), False, 10.0), ((8, 8, 16), False, 0.0), ((9, 9, 12), True, 20.0), ((41, 25, 1), True, 0.0)])
+def test_many_steps_match_two_launches_bitwise(L, open_ends, T, precision):
+    text = configs.sc_config(L=L, periodic=(not open_ends,) * 3, temperature=T, seed=9,
+                             precision=precision)
+    calls = (1, 2, 37, 1300)
+    for (a, ia, ma), (b, ib, mb) in zip(run(text, 0, calls), run(text, 256, calls)):
+        assert ia == ib
+        assert np.array_equal(a, b) and np.array_equal(ma, mb)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32-field"])
+def test_two_basis_sites_and_anisotropy(precision):
+    text = configs.c2(8, precision=precision)  # 1024 spins, two shells, K1, 300 K
+    for (a, _, _), (b, _, _) in zip(run(text, 0, (50, 3)), run(text, 256, (50, 3))):
+        assert np.array_equal(a, b)
+
+
+def test_injected_noise_and_free_spins_match_the_oracle(engine_factory):
+    n = 130
+    b = S.c1(6)
+    w = np.random.default_rng(4).standard_normal((b.n, 3))
+    e = b.engine(engine_factory)
+    e.set_noise(w)
+    e.step(20)
+    o, s = b.oracle(), b.s0.copy()
+    for k in range(20):
+        o.heun_step(s, b.dt, k * b.dt, w)
+    assert np.array_equal(e.get_spins(), s)
+    # no exchange at all
+    mus, gyro, alpha = np.full(n, 2.0 * S.BOHR), np.full(n, S.gyro_e()), np.full(n, 0.1)
+    dc = np.tile([0.1, 0.2, 1.0], (n, 1)) * mus[:, None]
+    e = engine_factory()
+    e.set_sites(mus, gyro, alpha)
+    e.add_zeeman(dc)
+    e.set_time_step(1e-3)
+    s = po.random_spins(2, n)
+    e.set_spins(s)
+    e.step(30)
+    o = po.OracleSystem(mus, gyro, alpha)
+    o.add_zeeman(dc)
+    for k in range(30):
+        o.heun_step(s, 1e-3, k * 1e-3)
+    assert np.array_equal(e.get_spins(), s)
