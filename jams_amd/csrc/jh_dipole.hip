@@ -54,6 +54,7 @@ constexpr double kMu0IU = 4.0 * kPi * 1e-7 / 6.24150907e21;  // helpers/consts.h
 constexpr double kDistTol = 1e-4;                              // helpers/defaults.h:44
 constexpr size_t kMaxPassLds = 64 * 1024;  // one line of the longest axis per workgroup
 constexpr int kMaxBasis = 8;
+constexpr int64_t kFusedBlocks = 512;  // workgroups of the fused x kernel, at least: two per CU
 
 #define DCHK(x)                              \
   do {                                       \
@@ -87,6 +88,33 @@ std::vector<int> factorise(int n) {
   for (int f : {5, 3}) while (n % f == 0) { r.push_back(f); n /= f; }
   for (int f = 7; n > 1; f += 2) while (n % f == 0) { r.push_back(f); n /= f; }
   return r;
+}
+
+// Radices of an axis of the fused kernels: the fewest of those they are built
+// for (then the smallest), since every stage costs two barriers and a trip
+// through LDS: 180 = 15 x 12, 150 = 15 x 10, 400 = 10 x 10 x 4 against 4 x 5 x
+// 3 x 3, 2 x 5 x 5 x 3 and 8 x 2 x 5 x 5.  512 stays 8 x 8 x 8, which has
+// stages of its own.  Empty when n has a prime factor above 7.
+std::vector<int> fused_radices(int n) {
+  static const int set[] = {16, 15, 12, 10, 9, 8, 7, 6, 5, 4, 3, 2};
+  std::vector<int> best;
+  int best_sum = 0;
+  for (int r : set) {
+    if (n % r) continue;
+    std::vector<int> s{r};
+    if (n > r) {
+      const std::vector<int> rest = fused_radices(n / r);
+      if (rest.empty()) continue;
+      s.insert(s.end(), rest.begin(), rest.end());
+    }
+    int sum = 0;
+    for (int q : s) sum += q;
+    if (best.empty() || s.size() < best.size() || (s.size() == best.size() && sum < best_sum)) {
+      best = s;
+      best_sum = sum;
+    }
+  }
+  return best;
 }
 
 // exp(-2 pi i t / n), t < n.  Entries of the first half are evaluated in long
@@ -170,6 +198,7 @@ struct XFused {
   int ns[fft::kMaxStages];
   float ns_rcp[fft::kMaxStages];
   int tws[fft::kMaxStages];
+  int m[fft::kMaxStages];  // butterflies per line, n / radix
   int L0;          // occupied x (inputs and outputs)
   int by, lby;     // y lines per workgroup, by = 1 << lby
   int lw;          // 3 by lines in LDS
@@ -189,7 +218,7 @@ __device__ __forceinline__ void xf_stage(const PP &p, const typename fft::C2<T>:
                                          typename fft::C2<T>::type *A, int st) {
   using T2 = typename fft::C2<T>::type;
   constexpr int NBF = fft::kBF<T, R>;
-  const int n = p.n, lw = p.lw, m = n / R, total = m * lw, nt = blockDim.x;
+  const int lw = p.lw, m = p.m[st], total = m * lw, nt = blockDim.x;
   const int Ns = p.ns[st], tws = p.tws[st];
   const float rns = p.ns_rcp[st];
   T2 v[NBF][R];
@@ -203,10 +232,14 @@ __device__ __forceinline__ void xf_stage(const PP &p, const typename fft::C2<T>:
       const int jd = fft::divmod_small(j, Ns, rns, jm);
       dq[q] = (jd * Ns * R + jm) * lw + l;
 #pragma unroll
-      for (int r = 0; r < R; ++r) v[q][r] = A[(j + r * m) * lw + l];
+      for (int r = 0; r < R; ++r) v[q][r] = A[t + r * total];
+      if (Ns > 1) {  // the first stage's twiddles are 1
+        const int dw = __mul24(jm, tws);
+        int w = dw;
 #pragma unroll
-      for (int r = 1; r < R; ++r) v[q][r] = fft::cmul(v[q][r], fft::twiddle<T, INV>(tw, jm * r * tws));
-      fft::dft_fixed<T2, R>(v[q], INV);
+        for (int r = 1; r < R; ++r, w += dw) v[q][r] = fft::cmul(v[q][r], fft::twiddle<T, INV>(tw, w));
+      }
+      fft::dft_any<T2, R, INV>(v[q]);
     }
   }
   __syncthreads();
@@ -230,7 +263,14 @@ __device__ __forceinline__ void xf_stages(const PP &p, const typename fft::C2<T>
       case 3: xf_stage<T, 3, INV>(p, tw, A, st); break;
       case 4: xf_stage<T, 4, INV>(p, tw, A, st); break;
       case 5: xf_stage<T, 5, INV>(p, tw, A, st); break;
-      default: xf_stage<T, 8, INV>(p, tw, A, st); break;
+      case 6: xf_stage<T, 6, INV>(p, tw, A, st); break;
+      case 7: xf_stage<T, 7, INV>(p, tw, A, st); break;
+      case 8: xf_stage<T, 8, INV>(p, tw, A, st); break;
+      case 9: xf_stage<T, 9, INV>(p, tw, A, st); break;
+      case 10: xf_stage<T, 10, INV>(p, tw, A, st); break;
+      case 12: xf_stage<T, 12, INV>(p, tw, A, st); break;
+      case 15: xf_stage<T, 15, INV>(p, tw, A, st); break;
+      default: xf_stage<T, 16, INV>(p, tw, A, st); break;
     }
   }
 }
@@ -294,6 +334,22 @@ __device__ __forceinline__ void xf_stages512(const typename fft::C2<T>::type *tw
   xf_stage512<T, 64, INV, LW>(tw, A, j, l);
 }
 
+// store(e, load(e)) for e = tid, tid + nt, ... < total, with the loads of U
+// elements of a thread in flight together (load must be valid for any e in
+// [0, total); the elements past the end repeat the last one)
+template <int U, class L, class S>
+__device__ __forceinline__ void batched(int total, L &&load, S &&store) {
+  const int nt = blockDim.x;
+  for (int e0 = threadIdx.x; e0 < total; e0 += U * nt) {
+    decltype(load(0)) v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) v[u] = load(min(e0 + u * nt, total - 1));
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (e0 + u * nt < total) store(e0 + u * nt, v[u]);
+  }
+}
+
 // e = q lw + l with a compile-time lw when LW > 0
 template <int LW>
 __device__ __forceinline__ int divmod_lw(int e, int lw, float rcp, int &l) {
@@ -329,15 +385,21 @@ __global__ void __launch_bounds__(512) k_dip_x_fused(const XFused<T> p) {
   const int64_t blk = xcd_block(blockIdx.x, gridDim.x);
   const int q2 = (int)(blk / p.nyb), y0 = (int)(blk % p.nyb) << lby;
   T2 *K = p.K + (int64_t)q2 * p.sq + y0;
-  // load x < L0 (zero padding above), element e = x lw + c by + yb
-  for (int e = threadIdx.x; e < n * lw; e += nt) {
-    int l;
-    const int x = divmod_lw<LWK>(e, lw, p.lw_rcp, l);
-    const int c = l >> lby, yb = l & (by - 1);
+  // load x < L0, element e = x lw + c by + yb, and pad with zeros above (a y
+  // line past the plane's end repeats the last one and is not stored)
+  batched<4>(
+      p.L0 * lw,
+      [&](int e) {
+        int l;
+        const int x = divmod_lw<LWK>(e, lw, p.lw_rcp, l);
+        const int c = l >> lby, yb = min(l & (by - 1), p.P1 - 1 - y0);
+        return K[c * p.M + (int64_t)x * p.P1 + yb];
+      },
+      [&](int e, T2 v) { A[e] = v; });
+  for (int e = p.L0 * lw + (int)threadIdx.x; e < n * lw; e += nt) {
     T2 v;
     v.x = 0;
     v.y = 0;
-    if (x < p.L0 && y0 + yb < p.P1) v = K[c * p.M + (int64_t)x * p.P1 + yb];
     A[e] = v;
   }
   __syncthreads();
@@ -346,19 +408,23 @@ __global__ void __launch_bounds__(512) k_dip_x_fused(const XFused<T> p) {
   {
     const int nby = n * by;
     const T *W = p.W + blk * 6 * nby;
-    for (int e = threadIdx.x; e < nby; e += nt) {
-      T2 *a = A + (e >> lby) * lw + (e & (by - 1));
-      const T2 sx = a[0], sy = a[by], sz = a[2 * by];
-      const T xx = W[e], xy = W[nby + e], xz = W[2 * nby + e], yy = W[3 * nby + e],
-              yz = W[4 * nby + e], zz = W[5 * nby + e];
-      T2 hx, hy, hz;
-      hx.x = xx * sx.x + xy * sy.x + xz * sz.x; hx.y = xx * sx.y + xy * sy.y + xz * sz.y;
-      hy.x = xy * sx.x + yy * sy.x + yz * sz.x; hy.y = xy * sx.y + yy * sy.y + yz * sz.y;
-      hz.x = xz * sx.x + yz * sy.x + zz * sz.x; hz.y = xz * sx.y + yz * sy.y + zz * sz.y;
-      a[0] = hx;
-      a[by] = hy;
-      a[2 * by] = hz;
-    }
+    struct Sym { T xx, xy, xz, yy, yz, zz; };
+    batched<2>(
+        nby,
+        [&](int e) {
+          return Sym{W[e], W[nby + e], W[2 * nby + e], W[3 * nby + e], W[4 * nby + e], W[5 * nby + e]};
+        },
+        [&](int e, const Sym &w) {
+          T2 *a = A + (e >> lby) * lw + (e & (by - 1));
+          const T2 sx = a[0], sy = a[by], sz = a[2 * by];
+          T2 hx, hy, hz;
+          hx.x = w.xx * sx.x + w.xy * sy.x + w.xz * sz.x; hx.y = w.xx * sx.y + w.xy * sy.y + w.xz * sz.y;
+          hy.x = w.xy * sx.x + w.yy * sy.x + w.yz * sz.x; hy.y = w.xy * sx.y + w.yy * sy.y + w.yz * sz.y;
+          hz.x = w.xz * sx.x + w.yz * sy.x + w.zz * sz.x; hz.y = w.xz * sx.y + w.yz * sy.y + w.zz * sz.y;
+          a[0] = hx;
+          a[by] = hy;
+          a[2 * by] = hz;
+        });
   }
   __syncthreads();
   line_stages<T, true, LWK>(p, tw, A);
@@ -639,6 +705,7 @@ struct ZYFused {
   int ns[fft::kMaxStages];
   float ns_rcp[fft::kMaxStages];
   int tws[fft::kMaxStages];
+  int m[fft::kMaxStages];
   int lw;          // q2 lines per workgroup
   float lw_rcp;
   int nsplit;      // workgroups per (g, x): q2 in [s lw, s lw + lw) ∩ [0, Q2)
@@ -674,22 +741,33 @@ __global__ void __launch_bounds__(512) k_dip_zy_fwd(const ZYFused<T> p) {
   const int L1 = p.L1, L2 = p.L2, SV = odd_stride(L2);
   // spins of cells (x, y < L1, z < L2), basis m, in memory order
   const int64_t base = (int64_t)x * L1 * L2 * p.nb + m;
-  for (int e = tid; e < L1 * L2; e += nt) {
-    const int64_t idx = base + (int64_t)e * p.nb;
-    // (y, z) of element e: a shift when L2 fills the register bound LM
-    const int y = L2 == LM ? e / LM : e / L2, z = e - y * L2;
-    vals[y * SV + z] = (T)(p.mus[idx] * p.spins[spin_idx(p.nspin, idx, comp)]);
-  }
+  batched<4>(
+      L1 * L2,
+      [&](int e) {
+        const int64_t idx = base + (int64_t)e * p.nb;
+        return (T)(p.mus[idx] * p.spins[spin_idx(p.nspin, idx, comp)]);
+      },
+      [&](int e, T v) {
+        // (y, z) of element e: a shift when L2 fills the register bound LM
+        const int y = L2 == LM ? e / LM : e / L2, z = e - y * L2;
+        vals[y * SV + z] = v;
+      });
   __syncthreads();
-  // direct DFT along z of line y (the arithmetic of k_dip_z_direct_fwd)
+  // direct DFT along z (the arithmetic of k_dip_z_direct_fwd): the threads
+  // take the cells (x, y), in as many groups as there are threads for, the
+  // groups the q2 lines in turn
+  // (512-point lines: one group, with the threads the butterflies need)
+  const int groups = LWK ? 1 : max(1, min(lw, nt / L1));
+  const int grp = LWK ? 0 : tid / L1, yc = tid - grp * L1;
+  const bool zlive = LWK ? tid < L1 : grp < groups;
   T v[LM];
-  if (tid < L1) {
+  if (zlive) {
 #pragma unroll
-    for (int z = 0; z < LM; ++z) v[z] = z < L2 ? vals[tid * SV + z] : (T)0;
+    for (int z = 0; z < LM; ++z) v[z] = z < L2 ? vals[yc * SV + z] : (T)0;
   }
   __syncthreads();  // vals is overwritten by A below
-  if (tid < L1) {
-    for (int l = 0; l < lw; ++l) {
+  if (zlive) {
+    for (int l = grp; l < lw; l += groups) {
       const int q = qa + l;
       T2 acc;
       acc.x = 0;
@@ -707,7 +785,7 @@ __global__ void __launch_bounds__(512) k_dip_zy_fwd(const ZYFused<T> p) {
           }
         }
       }
-      A[tid * lw + l] = acc;
+      A[yc * lw + l] = acc;
     }
   }
   // zero padding y >= L1
@@ -750,38 +828,47 @@ __global__ void __launch_bounds__(512) k_dip_zy_inv(const ZYFused<T> p) {
   const int x = (int)(blk % p.L0), g = (int)(blk / p.L0);
   const int m = g / 3, comp = g % 3;
   const T2 *K = p.K + (int64_t)g * p.sa + (int64_t)x * n;
-  // c2r sums of line y = tid: X[0] + 2 Re(X[k] w^{kz}) for 0 < k < P2/2
-  // (+ X[P2/2] (-1)^z, P2 even)
+  // c2r sums of the thread's cell: X[0] + 2 Re(X[k] w^{kz}) for 0 < k < P2/2
+  // (+ X[P2/2] (-1)^z, P2 even).  The threads take the cells (x, y), in as
+  // many groups as there are threads for, the groups every groups-th z
+  // (512-point lines: one group, with the threads the butterflies need)
+  const int groups = LWK ? 1 : max(1, min(L2, nt / L1));
+  const int grp = LWK ? 0 : tid / L1, yc = tid - grp * L1;
+  const bool zlive = LWK ? tid < L1 : grp < groups;
   T acc[LM];
   for (int q0 = 0; q0 < Q2; q0 += lw) {
     const int nq = min(lw, Q2 - q0);
-    for (int e = tid; e < n * lw; e += nt) {
-      const int l = e / n, y = e - l * n;
-      T2 v;
-      v.x = 0;
-      v.y = 0;
-      if (l < nq) v = K[(int64_t)(q0 + l) * p.sq + y];
-      A[y * lw + l] = v;
-    }
+    batched<4>(
+        n * lw,
+        [&](int e) {
+          const int l = e / n, y = e - l * n;
+          return K[(int64_t)(q0 + min(l, nq - 1)) * p.sq + y];
+        },
+        [&](int e, T2 v) {
+          const int l = e / n, y = e - l * n;
+          A[y * lw + l] = v;
+        });
     __syncthreads();
     line_stages<T, true, LWK>(p, twy, A);
-    if (tid < L1) {
+    if (zlive) {
       for (int l = 0; l < nq; ++l) {
         const int k = q0 + l;
-        const T2 X = A[tid * lw + l];
-        int t = 0;  // (k z) mod P2
+        const T2 X = A[yc * lw + l];
+        // (k z) mod P2 for z = grp, grp + groups, ...
+        int t = LWK ? 0 : (k * grp) % P2;
+        const int dt = LWK ? k : (k * groups) % P2;
 #pragma unroll
-        for (int z = 0; z < LM; ++z) {
-          if (z < L2) {
+        for (int i = 0; i < LM; ++i) {
+          if (grp + i * groups < L2) {
             if (k == 0) {
-              acc[z] = X.x;
+              acc[i] = X.x;
             } else {
               const T2 w = twz[t];  // e^{-2 pi i kz/P2}; conjugated below
               const T re = X.x * w.x + X.y * w.y;
-              if (2 * k == P2) acc[z] = acc[z] + re;
-              else acc[z] = acc[z] + 2 * re;
+              if (2 * k == P2) acc[i] = acc[i] + re;
+              else acc[i] = acc[i] + 2 * re;
             }
-            t += k;
+            t += dt;
             if (t >= P2) t -= P2;
           }
         }
@@ -789,18 +876,19 @@ __global__ void __launch_bounds__(512) k_dip_zy_inv(const ZYFused<T> p) {
     }
     __syncthreads();
   }
-  if (tid < L1) {
+  if (zlive) {
 #pragma unroll
-    for (int z = 0; z < LM; ++z)
-      if (z < L2) outs[tid * SZ + z] = acc[z];
+    for (int i = 0; i < LM; ++i)
+      if (grp + i * groups < L2) outs[yc * SZ + grp + i * groups] = acc[i];
   }
   __syncthreads();
   const int64_t base = (int64_t)x * L1 * L2 * p.nb + m;
-  for (int e = tid; e < L1 * L2; e += nt) {
-    const int y = L2 == LM ? e / LM : e / L2, z = e - y * L2;
-    const int64_t idx = base + (int64_t)e * p.nb;
-    p.field[comp * p.nspin + idx] = p.mus[idx] * (double)outs[y * SZ + z];
-  }
+  batched<4>(
+      L1 * L2, [&](int e) { return p.mus[base + (int64_t)e * p.nb]; },
+      [&](int e, double mus) {
+        const int y = L2 == LM ? e / LM : e / L2, z = e - y * L2;
+        p.field[comp * p.nspin + base + (int64_t)e * p.nb] = mus * (double)outs[y * SZ + z];
+      });
 }
 
 // tensor set-up: the q2 < Q2 half of the transformed grid into the tensor
@@ -923,7 +1011,8 @@ class DipoleFFTImpl : public DipoleFFT {
   int L[3], P[3], per[3], nb;
   int64_t n, Q2, M;  // M = P0 P1 Q2
   bool real_tensor = false;  // W(n) = W(-n): the transformed tensor is real
-  std::vector<int> rad[3];
+  std::vector<int> rad[3];   // the separate passes' radices
+  std::vector<int> frad[3];  // the fused kernels' (empty: not for them)
   DBuf<double> mus;
   Plane<double> f64;
   Plane<float> f32;
@@ -947,18 +1036,28 @@ class DipoleFFTImpl : public DipoleFFT {
     return p;
   }
 
+  // threads of a fused workgroup: what its butterflies need, and about one per
+  // four of the elements that it loads and stores, in whole sets of four waves
+  // beyond four (a 90 x 75 x 6 film's FP32 evaluation 30.9 -> 27.5 us, a 64 x
+  // 64 x 8 one's FP64 34.2 -> 29.8; with five waves, which put two on one SIMD
+  // unit, a 200 x 200 x 8 film's z + y forward kernel took 42 us, with four
+  // 26).  512-point lines keep their butterflies' count.
+  static int fused_threads(int need, int n, int lw) {
+    if (n != 512) {
+      int want = std::min(512, n * lw / 4);
+      if (want > 256) want -= want % 256;
+      need = std::max(need, want);
+    }
+    return (need + 63) / 64 * 64;
+  }
   // threads of the fused x kernel for by y lines: enough that no thread
   // holds more than kBF butterflies of any stage
   template <class T>
   int xf_threads(int by) const {
     const int n = P[0], lw = 3 * by;
     int need = 64;
-    for (int R : rad[0]) {
-      const int kbf = R == 2 ? fft::kBF<T, 2> : R == 3 ? fft::kBF<T, 3> : R == 4 ? fft::kBF<T, 4>
-                    : R == 5 ? fft::kBF<T, 5> : fft::kBF<T, 8>;
-      need = std::max(need, (n / R * lw + kbf - 1) / kbf);
-    }
-    return (need + 63) / 64 * 64;
+    for (int R : frad[0]) need = std::max(need, (n / R * lw + fft::kbf_of(R) - 1) / fft::kbf_of(R));
+    return fused_threads(need, n, lw);
   }
   // axis of 512 points factored 8 x 8 x 8: the fused kernels' compile-time
   // stage geometry applies
@@ -971,16 +1070,19 @@ class DipoleFFTImpl : public DipoleFFT {
 
   // y lines per workgroup of the fused x kernel (0: not applicable): one
   // basis site with a real tensor, in-place radices, LDS within 64 KB (two
-  // workgroups per CU), at most 512 threads
+  // workgroups per CU), at most 512 threads; fewer lines, down to 2, where
+  // the grid would otherwise leave compute units idle
   template <class T>
   int fused_lines() const {
-    if (nb != 1 || !real_tensor) return 0;
-    for (int r : rad[0])
-      if (r != 2 && r != 3 && r != 4 && r != 5 && r != 8) return 0;
+    if (nb != 1 || !real_tensor || frad[0].empty()) return 0;
     const size_t c = sizeof(typename fft::C2<T>::type);
-    for (int by = 8; by >= 1; by /= 2)
-      if ((size_t)P[0] * (3 * by + 1) * c <= kMaxPassLds && xf_threads<T>(by) <= 512) return by;
-    return 0;
+    int fit = 0;
+    for (int by = 8; by >= 1; by /= 2) {
+      if ((size_t)P[0] * (3 * by + 1) * c > kMaxPassLds || xf_threads<T>(by) > 512) continue;
+      fit = by;
+      if (by <= 2 || Q2 * ((P[1] + by - 1) / by) >= kFusedBlocks) break;
+    }
+    return fit;
   }
 
   template <class T>
@@ -989,10 +1091,11 @@ class DipoleFFTImpl : public DipoleFFT {
     XFused<T> q;
     std::memset(&q, 0, sizeof q);
     q.n = P[0];
-    q.nst = (int)rad[0].size();
+    q.nst = (int)frad[0].size();
     int Ns = 1;
     for (int k = 0; k < q.nst; ++k) {
-      q.radix[k] = rad[0][k];
+      q.radix[k] = frad[0][k];
+      q.m[k] = q.n / q.radix[k];
       q.ns[k] = Ns;
       q.ns_rcp[k] = 1.0f / (float)Ns;
       q.tws[k] = q.n / (Ns * q.radix[k]);
@@ -1112,12 +1215,8 @@ class DipoleFFTImpl : public DipoleFFT {
   template <class T>
   int zy_threads(int lw) const {
     int need = std::max(64, L[1]);
-    for (int R : rad[1]) {
-      const int kbf = R == 2 ? fft::kBF<T, 2> : R == 3 ? fft::kBF<T, 3> : R == 4 ? fft::kBF<T, 4>
-                    : R == 5 ? fft::kBF<T, 5> : fft::kBF<T, 8>;
-      need = std::max(need, (P[1] / R * lw + kbf - 1) / kbf);
-    }
-    return (need + 63) / 64 * 64;
+    for (int R : frad[1]) need = std::max(need, (P[1] / R * lw + fft::kbf_of(R) - 1) / fft::kbf_of(R));
+    return fused_threads(need, P[1], lw);
   }
   template <class T>
   size_t zy_lds(int lw) const {
@@ -1133,9 +1232,7 @@ class DipoleFFTImpl : public DipoleFFT {
   // than 5 or 2)
   template <class T>
   int zy_split() const {
-    if (!direct_z()) return 0;
-    for (int r : rad[1])
-      if (r != 2 && r != 3 && r != 4 && r != 5 && r != 8) return 0;
+    if (!direct_z() || frad[1].empty()) return 0;
     for (int ns = Q2 >= 4 ? JH_ZY_SPLIT : 1; ns <= Q2; ++ns) {
       const int lw = (int)((Q2 + ns - 1) / ns);
       if (zy_lds<T>(lw) <= kMaxPassLds && zy_threads<T>(lw) <= 512) return ns;
@@ -1168,10 +1265,11 @@ class DipoleFFTImpl : public DipoleFFT {
     ZYFused<T> q;
     std::memset(&q, 0, sizeof q);
     q.n = P[1];
-    q.nst = (int)rad[1].size();
+    q.nst = (int)frad[1].size();
     int Ns = 1;
     for (int k = 0; k < q.nst; ++k) {
-      q.radix[k] = rad[1][k];
+      q.radix[k] = frad[1][k];
+      q.m[k] = q.n / q.radix[k];
       q.ns[k] = Ns;
       q.ns_rcp[k] = 1.0f / (float)Ns;
       q.tws[k] = q.n / (Ns * q.radix[k]);
@@ -1406,6 +1504,7 @@ DipoleFFT *DipoleFFT::create(const int32_t size[3], const int32_t periodic[3], i
     if (pass_lds<double>(d->P[a], 1, true) > kMaxPassLds)
       return fail("padded dimension too long for one workgroup's LDS (at most 2048)");
     d->rad[a] = factorise(d->P[a]);
+    d->frad[a] = d->P[a] == 512 ? d->rad[a] : fused_radices(d->P[a]);
     if ((int)d->rad[a].size() > fft::kMaxStages) return fail("too many FFT stages");
     for (int r : d->rad[a])
       if (r > 64) return fail("padded dimension has a prime factor above 64");

@@ -21,6 +21,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <utility>
+
 #include "jh_layout.h"
 
 // The transforms need no particular rounding sequence (the dipole's parity is
@@ -184,6 +186,123 @@ __device__ __forceinline__ void dft_fixed(T2 *v, bool inv) {
   }
 }
 
+// cos and sin of 2 pi t / N at compile time (Taylor series of the angle
+// reduced to [-pi, pi], in long double)
+constexpr long double root_angle(int t, int N) {
+  const int r = ((t % N) + N) % N;
+  const int q = 2 * r > N ? r - N : r;
+  return 2.0L * 3.141592653589793238462643383279502884L * q / N;
+}
+constexpr double root_cos(int t, int N) {
+  const long double x = root_angle(t, N);
+  long double term = 1.0L, sum = 1.0L;
+  for (int k = 1; k <= 20; ++k) {
+    term *= -x * x / ((2 * k - 1) * (2 * k));
+    sum += term;
+  }
+  return (double)sum;
+}
+constexpr double root_sin(int t, int N) {
+  const long double x = root_angle(t, N);
+  long double term = x, sum = x;
+  for (int k = 1; k <= 20; ++k) {
+    term *= -x * x / ((2 * k) * (2 * k + 1));
+    sum += term;
+  }
+  return (double)sum;
+}
+
+template <class F, int... I>
+__device__ __forceinline__ void static_for_impl(F &&f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void static_for(F &&f) {
+  static_for_impl(f, std::make_integer_sequence<int, N>{});
+}
+
+// R = R1 * R2 as nested DFTs: X[k1 + R1 k2] = sum_n2 w_R2^(n2 k2) w_R^(n2 k1)
+// sum_n1 w_R1^(n1 k1) x[R2 n1 + n2]
+template <class T2, int R, bool INV>
+__device__ __forceinline__ void dft_any(T2 *v);
+template <class T2, int R1, int R2, bool INV>
+__device__ __forceinline__ void dft_nested(T2 *v) {
+  using T = typename Re<T2>::type;
+  constexpr int R = R1 * R2;
+  T2 y[R];
+  static_for<R2>([&](auto n2c) {
+    constexpr int n2 = decltype(n2c)::value;
+    T2 a[R1];
+#pragma unroll
+    for (int n1 = 0; n1 < R1; ++n1) a[n1] = v[R2 * n1 + n2];
+    dft_any<T2, R1, INV>(a);
+    y[n2] = a[0];
+    static_for<R1 - 1>([&](auto kc) {
+      constexpr int k1 = decltype(kc)::value + 1;
+      if constexpr (n2 == 0) {
+        y[k1 * R2] = a[k1];
+      } else {
+        constexpr double c = root_cos(n2 * k1, R);
+        constexpr double s = (INV ? 1.0 : -1.0) * root_sin(n2 * k1, R);
+        T2 w;
+        w.x = (T)c;
+        w.y = (T)s;
+        y[k1 * R2 + n2] = cmul(a[k1], w);
+      }
+    });
+  });
+#pragma unroll
+  for (int k1 = 0; k1 < R1; ++k1) {
+    dft_any<T2, R2, INV>(y + k1 * R2);
+#pragma unroll
+    for (int k2 = 0; k2 < R2; ++k2) v[k1 + R1 * k2] = y[k1 * R2 + k2];
+  }
+}
+template <class T2, int R, bool INV>
+__device__ __forceinline__ void dft_any(T2 *v) {
+  using T = typename Re<T2>::type;
+  if constexpr (R == 6) dft_nested<T2, 2, 3, INV>(v);
+  else if constexpr (R == 9) dft_nested<T2, 3, 3, INV>(v);
+  else if constexpr (R == 10) dft_nested<T2, 2, 5, INV>(v);
+  else if constexpr (R == 12) dft_nested<T2, 4, 3, INV>(v);
+  else if constexpr (R == 15) dft_nested<T2, 5, 3, INV>(v);
+  else if constexpr (R == 16) dft_nested<T2, 4, 4, INV>(v);
+  else if constexpr (R == 7) {
+    // X[k], X[7 - k] = x0 + sum_q cos(2 pi q k / 7) t_q -+ i sum_q sin(..) u_q,
+    // t_q = x_q + x_(7-q), u_q = x_q - x_(7-q)
+    T2 t[3], u[3];
+    T2 x0 = v[0], s0 = v[0];
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      t[q] = cadd(v[q + 1], v[6 - q]);
+      u[q] = csub(v[q + 1], v[6 - q]);
+      s0 = cadd(s0, t[q]);
+    }
+    v[0] = s0;
+    static_for<3>([&](auto kc) {
+      constexpr int k = decltype(kc)::value + 1;
+      T2 e = x0, o;
+      o.x = 0;
+      o.y = 0;
+      static_for<3>([&](auto qc) {
+        constexpr int q = decltype(qc)::value + 1;
+        constexpr double c = root_cos(q * k, 7);
+        constexpr double s = (INV ? 1.0 : -1.0) * root_sin(q * k, 7);
+        e.x += (T)c * t[q - 1].x;
+        e.y += (T)c * t[q - 1].y;
+        o.x += (T)s * u[q - 1].x;
+        o.y += (T)s * u[q - 1].y;
+      });
+      v[k].x = e.x - o.y;
+      v[k].y = e.y + o.x;
+      v[7 - k].x = e.x + o.y;
+      v[7 - k].y = e.y - o.x;
+    });
+  } else {
+    dft_fixed<T2, R>(v, INV);
+  }
+}
+
 // q = x / d and r = x % d for 0 <= x < 2^22, 1 <= d < 2^22, with rd the
 // float nearest 1/d: the float estimate is within one of the quotient, and
 // one correction step makes it exact (no integer division instruction).
@@ -237,8 +356,9 @@ __device__ __forceinline__ void stage_fixed(const Pass<T> &p, const typename C2<
 // Butterflies per thread of an in-place stage: R * kBF <= 8 complex values
 // in registers (with 16, the 512-thread workgroups hold 108-188 VGPRs and one
 // fits per CU; with 8, two do, and the passes run 25-30 % faster).
+constexpr int kbf_of(int R) { return R <= 8 ? 8 / R : 1; }
 template <class T, int R>
-constexpr int kBF = (8 / R) > 0 ? 8 / R : 1;
+constexpr int kBF = kbf_of(R);
 
 // The same stage in place on one LDS buffer: every thread first reads and
 // transforms its butterflies (at most kBF<T, R>, which the host guarantees by
