@@ -84,6 +84,16 @@ constexpr int64_t kLnAutoMinRow = 24;           // neighbours per row from which
 // typically about a second, against a phase of under a millisecond for a few
 // million spins
 constexpr unsigned kStepPollLimit = 1u << 20;
+// Small contexts replay a captured graph of kAutoGraphSteps steps by
+// themselves, once they have run kAutoGraphAfter steps since they were laid
+// out: a launch in a graph costs the GPU about 0.8 us less than a plain one (sc
+// 16^3 thermal 11.9 -> 10.1 us per step, bcc 32^3 x 2 14.0 -> 12.3, a random
+// alloy of 152 k spins 17.8 -> 16.4; bcc 64^3 x 2 gains nothing and keeps plain
+// launches), but building it takes 0.3 to 0.6 ms, which a short run would not
+// win back.
+constexpr int kAutoGraphSteps = 20;
+constexpr int64_t kAutoGraphAfter = 500;
+constexpr int64_t kAutoGraphSpins = (int64_t)1 << 18;
 // steps of one launch of k_heun_many (a few ms at most)
 constexpr int kManyStepsMax = 1024;
 // vector operations per step (spins x operations per spin) up to which
@@ -368,7 +378,10 @@ struct jh_ctx {
   int step_launch = JH_STEP_LAUNCH_TWO;
   DevBuf<unsigned> step_sync;
   int cus = 0;
-  int graph_steps = 0;              // steps per captured graph (0: plain launches)
+  int graph_steps = 0;              // steps per captured graph (0: plain launches,
+                                    // or the engine's own choice, auto_graph)
+  bool auto_graph = true;
+  int64_t steps_run = 0;            // plain steps since the last layout
   hipGraph_t graph = nullptr;
   hipGraphExec_t gexec = nullptr;
   DevBuf<uint64_t> dstep;
@@ -1884,6 +1897,7 @@ void prepare(jh_ctx *c) {
   }
   sync_f32(c);
   HIPCHK(hipStreamSynchronize(c->stream));
+  c->steps_run = 0;
   c->dirty = false;
 }
 
@@ -2045,18 +2059,18 @@ void enqueue_step(jh_ctx *c, KParams p) {
   launch_phase(c, p, 1);
 }
 
-// Capture graph_steps steps.  Their kernels read the step counter as
+// Capture `steps` steps.  Their kernels read the step counter as
 // *c->dstep + k (k, the step's place in the graph, is baked into its
 // parameters), and the host sets *c->dstep once per replay with a one-thread
 // kernel outside the graph (no memset nodes).
-void build_graph(jh_ctx *c) {
+void build_graph(jh_ctx *c, int steps) {
   c->drop_graph();
   if (!c->dstep.p) c->dstep.alloc(1);
   KParams p = make_params(c);
   p.dstep = c->dstep.p;
   HIPCHK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
   try {
-    for (int k = 0; k < c->graph_steps; ++k) {
+    for (int k = 0; k < steps; ++k) {
       p.step = (uint64_t)k;
       enqueue_step(c, p);
     }
@@ -2083,6 +2097,14 @@ bool many_steps(const jh_ctx *c) {
   return (double)c->n * ops < kManyOps;
 }
 
+// steps per graph that a context without jh_set_graph_steps replays (0: none)
+int auto_graph_steps(const jh_ctx *c) {
+  return c->auto_graph && c->n <= kAutoGraphSpins && c->steps_run >= kAutoGraphAfter &&
+                 c->step_launch == JH_STEP_LAUNCH_TWO
+             ? kAutoGraphSteps
+             : 0;
+}
+
 void do_steps(jh_ctx *c, int64_t nsteps) {
   int64_t done = 0;
   if (many_steps(c)) {
@@ -2098,15 +2120,17 @@ void do_steps(jh_ctx *c, int64_t nsteps) {
     }
     return;
   }
-  if (c->graph_steps > 0 && nsteps >= c->graph_steps) {
-    if (!c->gexec) build_graph(c);
-    for (; done + c->graph_steps <= nsteps; done += c->graph_steps) {
+  const int graph_steps = c->graph_steps > 0 ? c->graph_steps : auto_graph_steps(c);
+  if (graph_steps > 0 && nsteps >= graph_steps) {
+    if (!c->gexec) build_graph(c, graph_steps);
+    for (; done + graph_steps <= nsteps; done += graph_steps) {
       HIPCHK(launch_set_step(c->dstep.p, (uint64_t)(c->iteration + done), c->stream));
       HIPCHK(hipGraphLaunch(c->gexec, c->stream));
     }
     c->iteration += done;
     c->time = (double)c->iteration * c->dt;
   }
+  c->steps_run += nsteps - done;
   KParams p = make_params(c);
   for (; done < nsteps; ++done) {
     p.step = (uint64_t)c->iteration;
@@ -2423,6 +2447,7 @@ int jh_set_noise(jh_ctx *c, const double *w) {
     c->winj.alloc((size_t)(3 * c->n));
     upload_vec(c, w, c->winj.p, false);
     c->noise_mode = NM_INJECTED;
+    c->drop_graph();  // its kernels hold the noise mode and buffer
   });
 }
 
@@ -2779,6 +2804,7 @@ int jh_autotune(jh_ctx *c, int steps, char *report, int64_t len) {
     const double t0 = c->time;
     const int fmt0 = c->xfmt_req, bs0 = c->block, gs0 = c->graph_steps, sl0 = c->step_launch;
     c->graph_steps = 0;
+    c->auto_graph = false;  // the candidates change the launches without a new layout
     c->step_launch = JH_STEP_LAUNCH_TWO;
     std::string rep;
     double best = 1e300;
@@ -2847,6 +2873,7 @@ int jh_autotune(jh_ctx *c, int steps, char *report, int64_t len) {
     c->block = best_bs;
     c->step_launch = best_sl;
     c->graph_steps = gs0;
+    c->auto_graph = true;
     c->dirty = true;
     prepare(c);
     HIPCHK(hipMemcpyAsync(c->s.p, save.p, sizeof(double) * 3 * c->n, hipMemcpyDeviceToDevice, c->stream));

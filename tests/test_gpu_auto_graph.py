@@ -1,0 +1,55 @@
+"""Small contexts replay a captured graph of their own accord after enough
+plain steps: the same bits as calls too short for a replay, replay after
+replay, with reductions, field evaluations and set-up changes in between."""
+import numpy as np
+import pytest
+
+from jams_amd import configs
+from jams_amd.host import Simulation
+
+pytestmark = pytest.mark.gpu
+
+F32 = "fp32-field"
+CASES = {
+    "heun": configs.sc_config(L=(13, 11, 12), temperature=20.0, seed=3),
+    "heun fp32": configs.sc_config(L=(13, 11, 12), temperature=20.0, seed=3, precision=F32),
+    "rk4": configs.bcc_config(L=9, seed=5).replace("llg-heun-gpu", "llg-rk4-gpu"),
+    "two shells": configs.bcc_config(L=9, seed=5),
+    "film": configs.sc_config(L=(14, 10, 3), periodic=(False,) * 3, field=None, dipole_rcut=20.0,
+                              alpha=0.02),
+    "film fp32": configs.sc_config(L=(14, 10, 3), periodic=(False,) * 3, field=None,
+                                   dipole_rcut=20.0, alpha=0.02, precision=F32),
+}
+
+
+def steps(e, n, most):
+    while n > 0:
+        e.step(min(n, most))
+        n -= most
+
+
+@pytest.mark.parametrize("name", CASES)
+def test_replays_match_short_calls_bitwise(name):
+    sims = [Simulation(CASES[name], device=0, output_dir="/tmp") for _ in range(2)]
+    a, b = (s.engine() for s in sims)
+    for k, n in enumerate((510, 100, 7, 45, 200)):
+        steps(a, n, 19)      # shorter than a replay: plain launches
+        steps(b, n, 10_000)
+        assert a.iteration() == b.iteration()
+        assert np.array_equal(a.get_spins(), b.get_spins()), (name, k)
+        assert np.array_equal(a.magnetisation(), b.magnetisation())
+        b.fields()
+        b.magnetisation()
+    # injected noise replaces the stream that the graph holds
+    w = np.random.default_rng(1).standard_normal((a.n, 3))
+    for e, most in ((a, 19), (b, 10_000)):
+        e.set_noise(w)
+        steps(e, 60, most)
+    assert np.array_equal(a.get_spins(), b.get_spins())
+    # and so does a new time step
+    for e, most in ((a, 19), (b, 10_000)):
+        e.set_time_step(5e-4)
+        steps(e, 560, most)
+    assert np.array_equal(a.get_spins(), b.get_spins())
+    for s in sims:
+        s.close()
