@@ -1483,8 +1483,16 @@ __device__ __forceinline__ void ln_field(const LnView &ln, int sid, int xw, int 
 #ifndef JH_LN_PRED_WAVES
 #define JH_LN_PRED_WAVES 5
 #endif
-template <int PHASE>
-constexpr int kLnWaves = PHASE == 0 ? JH_LN_PRED_WAVES : 1;
+// With one cell per lane (P = 1) the FP64 corrector fits 6 in 77 VGPRs without a
+// spill, where it would take 125 and 4 waves: five shells, 64^3 x 2 59.3 -> 51.9
+// us, step of 45^2 x 64 x 2 75.9 -> 66.8, of 16^2 x 64 x 2 48.5 -> 43.3.  At 8 it
+// spills 16: 50.5 us at 64^3 x 2, but slower on smaller lattices (16^2 x 64 x 2
+// 19.6 -> 27.7), and the FP32-field corrector the same (26.1 instead of 27.9 at
+// 64^3 x 2, 11.9 instead of 11.2 at 32^2 x 64 x 2).  The predictors are the same
+// at 5, 6 and 8.  With two cells per lane a cap costs more than it gives (128^3 x
+// 2, FP32-field step 326 us without, 377 at 5 and 455 at 6 waves).
+template <int PHASE, int P>
+constexpr int kLnWaves = PHASE == 0 ? JH_LN_PRED_WAVES : P == 1 ? 6 : 1;
 // The corrector's own s, ds and noise: read before the field (FP32-field
 // form: it forms s* from them) or after it (FP64, fewer live registers)
 #ifndef JH_LN_EARLY64
@@ -1496,7 +1504,7 @@ constexpr bool kLnEarlyOwn = kEarlyOwn<PREC> || JH_LN_EARLY64;
 // constant 0 and its parameters are read through the scalar unit.
 template <int PREC, bool DIAG, int PHASE, bool GEN, int P, bool ONE>
 __global__ void __launch_bounds__(kLnBlock)
-__attribute__((amdgpu_waves_per_eu(kLnWaves<PHASE>))) k_heun_ln(const KParams p, const LnView ln) {
+__attribute__((amdgpu_waves_per_eu(kLnWaves<PHASE, P>))) k_heun_ln(const KParams p, const LnView ln) {
   const int rlb = ln.rlblocks;
   if ((int)blockIdx.x < rlb) {
     // FP64 row list: the rows whose z neighbours wrap, each summed in its own
