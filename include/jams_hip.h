@@ -228,10 +228,14 @@ int jh_reduce_magnetisation_replicas(jh_ctx *ctx, double *out);
 
 /* ---- launch shape -------------------------------------------------------- */
 /* Run jh_step as replays of one captured hipGraph of `steps` Heun steps
- * (whatever is left over runs as plain launches); 0 disables graphs. */
+ * (whatever is left over runs as plain launches); 0 disables graphs.  Without
+ * a call, contexts of up to 2^18 spins replay a 20-step graph of their own
+ * once they have run 500 steps, with the same results. */
 int jh_set_graph_steps(jh_ctx *ctx, int steps);
 /* Threads per workgroup of the step kernels: 64 .. 512, a multiple of 64;
- * 0 (the default) picks 256 or 512 by exchange format. */
+ * 0 (the default) picks 256 or 512 by exchange format, and lets a context of
+ * up to 1024 spins run many steps per launch in one workgroup of its own
+ * size (same results). */
 int jh_set_block_size(jh_ctx *ctx, int threads);
 /* How jh_step launches a Heun step.  JH_STEP_LAUNCH_TWO (the default): a
  * predictor and a corrector launch, as the reference's step launches
