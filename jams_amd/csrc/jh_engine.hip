@@ -87,10 +87,10 @@ constexpr unsigned kStepPollLimit = 1u << 20;
 // Small contexts replay a captured graph of kAutoGraphSteps steps by
 // themselves, once they have run kAutoGraphAfter steps since they were laid
 // out: a launch in a graph costs the GPU about 0.8 us less than a plain one (sc
-// 16^3 thermal 11.9 -> 10.1 us per step, bcc 32^3 x 2 14.0 -> 12.3, a random
-// alloy of 152 k spins 17.8 -> 16.4; bcc 64^3 x 2 gains nothing and keeps plain
-// launches), but building it takes 0.3 to 0.6 ms, which a short run would not
-// win back.
+// 16^3 thermal 11.9 -> 10.1 us per step, bcc 32^3 x 2 14.0 -> 12.3; bcc 64^3 x 2
+// gains nothing and keeps plain launches), but building it takes 0.3 to 0.6 ms,
+// which a short run would not win back.  A call of jh_set_graph_steps takes the
+// choice over.
 constexpr int kAutoGraphSteps = 20;
 constexpr int64_t kAutoGraphAfter = 500;
 constexpr int64_t kAutoGraphSpins = (int64_t)1 << 18;
@@ -2777,6 +2777,7 @@ int jh_set_graph_steps(jh_ctx *c, int steps) {
   return guarded(c, [&] {
     if (steps < 0) JH_THROW(JH_ERR_INVALID, "steps must be >= 0");
     c->graph_steps = steps;
+    c->auto_graph = false;  // the caller chose, 0 included: no graph then
     c->drop_graph();
   });
 }
@@ -2804,6 +2805,7 @@ int jh_autotune(jh_ctx *c, int steps, char *report, int64_t len) {
     const double t0 = c->time;
     const int fmt0 = c->xfmt_req, bs0 = c->block, gs0 = c->graph_steps, sl0 = c->step_launch;
     c->graph_steps = 0;
+    const bool ag0 = c->auto_graph;
     c->auto_graph = false;  // the candidates change the launches without a new layout
     c->step_launch = JH_STEP_LAUNCH_TWO;
     std::string rep;
@@ -2873,7 +2875,7 @@ int jh_autotune(jh_ctx *c, int steps, char *report, int64_t len) {
     c->block = best_bs;
     c->step_launch = best_sl;
     c->graph_steps = gs0;
-    c->auto_graph = true;
+    c->auto_graph = ag0;
     c->dirty = true;
     prepare(c);
     HIPCHK(hipMemcpyAsync(c->s.p, save.p, sizeof(double) * 3 * c->n, hipMemcpyDeviceToDevice, c->stream));
