@@ -386,7 +386,9 @@ struct jh_ctx {
   hipGraphExec_t gexec = nullptr;
   DevBuf<uint64_t> dstep;
 
+  // replays may still be queued: jh_step does not wait for its launches
   void drop_graph() {
+    if (gexec) (void)hipStreamSynchronize(stream);
     if (gexec) (void)hipGraphExecDestroy(gexec);
     if (graph) (void)hipGraphDestroy(graph);
     gexec = nullptr;
@@ -1836,6 +1838,8 @@ void prepare(jh_ctx *c) {
   require_sites(c);
   if (!c->spins_set) JH_THROW(JH_ERR_STATE, "spins have not been set (jh_set_spins)");
   if (!c->dirty) return;
+  // steps may still be running: the tables that they read are overwritten below
+  HIPCHK(hipStreamSynchronize(c->stream));
   if (c->xh.size() > 1)
     JH_THROW(JH_ERR_UNSUPPORTED, "more than one exchange term; merge them into one list");
   int nzee = 0, nani = 0;
