@@ -906,6 +906,17 @@ k_heun_step(const KParams p, unsigned *sync, unsigned limit) {
   }
 }
 
+// LDS bytes of one of k_heun_many's two spin arrays: whole 16-byte words, since
+// the (x, y) pairs of both are read and written as such for odd n too
+__host__ __device__ constexpr size_t many_spin_bytes(int prec, int64_t n) {
+  return ((size_t)n * (prec == PR_FP64 ? 3 * sizeof(double) : kG32 * sizeof(float)) + 15) &
+         ~(size_t)15;
+}
+static_assert(many_spin_bytes(PR_FP64, 27) % sizeof(double2) == 0 &&
+                  many_spin_bytes(PR_FP64, 27) >= 27 * 3 * sizeof(double) &&
+                  many_spin_bytes(PR_FP32, 27) % sizeof(float4) == 0,
+              "the second array of an odd number of spins starts on a 16-byte word");
+
 // Many Heun steps of a small system in one launch of one workgroup: the spins
 // stay in LDS (s and s*, in the layout of the device arrays, or the FP32 form's
 // copies), each thread's own spin, ds and noise in registers, and a phase ends
@@ -921,8 +932,9 @@ __global__ void __launch_bounds__(kManySpins) k_heun_many(const KParams p, int n
   extern __shared__ __align__(16) unsigned char lds[];
   const int64_t n = p.n, i = threadIdx.x;
   const bool live = i < n;
-  double *A = reinterpret_cast<double *>(lds + lds_spins), *B = A + 3 * n;
-  float *A32 = reinterpret_cast<float *>(A), *B32 = A32 + (size_t)kG32 * n;
+  unsigned char *const a = lds + lds_spins, *const b = a + many_spin_bytes(PREC, n);
+  double *A = reinterpret_cast<double *>(a), *B = reinterpret_cast<double *>(b);
+  float *A32 = reinterpret_cast<float *>(a), *B32 = reinterpret_cast<float *>(b);
   auto put = [&](double *a, float *a32, const double (&v)[3]) {
     if constexpr (PREC == PR_FP64) store_spin(a, n, i, v[0], v[1], v[2]);
     else store_g32(a32, i, v[0], v[1], v[2]);
@@ -2039,7 +2051,7 @@ hipError_t launch_heun(const KParams &p, int prec, int xv, int phase, int bs, hi
 template <int PREC, int XVk>
 static hipError_t launch_heun_many_t(const KParams &p, int nsteps, hipStream_t st) {
   const int off = (int)((table_lds(p, PREC, XVk) + 15) & ~(size_t)15);
-  const size_t lds = off + 2 * (size_t)p.n * (PREC == PR_FP64 ? 3 * sizeof(double) : kG32 * sizeof(float));
+  const size_t lds = off + 2 * many_spin_bytes(PREC, p.n);
   const int threads = (int)((p.n + 63) / 64 * 64);
   const auto fn = k_heun_many<PREC, XVk>;
   if (lds > 64 * 1024) {

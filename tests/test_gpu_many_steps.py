@@ -71,3 +71,13 @@ def test_injected_noise_and_free_spins_match_the_oracle(engine_factory):
     for k in range(30):
         o.heun_step(s, 1e-3, k * 1e-3)
     assert np.array_equal(e.get_spins(), s)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32-field"])
+@pytest.mark.parametrize("L", [(3, 3, 3), (7, 7, 7), (9, 9, 9), (1023, 1, 1)])
+def test_odd_numbers_of_spins(L, precision):
+    """the second spin array in LDS starts behind an odd number of spins"""
+    text = configs.sc_config(L=L, periodic=(False,) * 3, temperature=20.0, seed=2,
+                             precision=precision)
+    for (a, _, ma), (b, _, mb) in zip(run(text, 0, (1, 60)), run(text, 128, (1, 60))):
+        assert np.array_equal(a, b) and np.array_equal(ma, mb)
