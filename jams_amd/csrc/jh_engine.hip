@@ -2124,9 +2124,20 @@ void do_steps(jh_ctx *c, int64_t nsteps) {
     }
     return;
   }
-  const int graph_steps = c->graph_steps > 0 ? c->graph_steps : auto_graph_steps(c);
+  int graph_steps = c->graph_steps > 0 ? c->graph_steps : auto_graph_steps(c);
+  if (graph_steps > 0 && nsteps >= graph_steps && !c->gexec) {
+    try {
+      build_graph(c, graph_steps);
+    } catch (const JhError &) {
+      if (c->graph_steps > 0) throw;
+      // nobody asked for this graph: plain launches from here on
+      c->drop_graph();
+      (void)hipGetLastError();
+      c->auto_graph = false;
+      graph_steps = 0;
+    }
+  }
   if (graph_steps > 0 && nsteps >= graph_steps) {
-    if (!c->gexec) build_graph(c, graph_steps);
     for (; done + graph_steps <= nsteps; done += graph_steps) {
       HIPCHK(launch_set_step(c->dstep.p, (uint64_t)(c->iteration + done), c->stream));
       HIPCHK(hipGraphLaunch(c->gexec, c->stream));

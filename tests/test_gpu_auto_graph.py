@@ -1,6 +1,10 @@
 """Small contexts replay a captured graph of their own accord after enough
 plain steps: the same bits as calls too short for a replay, replay after
 replay, with reductions, field evaluations and set-up changes in between."""
+import subprocess
+import sys
+from pathlib import Path
+
 import numpy as np
 import pytest
 
@@ -53,3 +57,39 @@ def test_replays_match_short_calls_bitwise(name):
     assert np.array_equal(a.get_spins(), b.get_spins())
     for s in sims:
         s.close()
+
+
+CHILD = """
+import ctypes, sys
+ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)  # before the engine's own HIP library
+import numpy as np
+from jams_amd import configs
+from jams_amd.engine import EngineError
+from jams_amd.host import Simulation
+a, b = (Simulation(configs.c1(16, temperature=10.0), device=0, output_dir="/tmp") for _ in range(2))
+for s, most in ((a, 19), (b, 700)):
+    e, n = s.engine(), 1400
+    while n > 0:
+        e.step(min(n, most))
+        n -= most
+assert np.array_equal(a.engine().get_spins(), b.engine().get_spins())
+e = a.engine()
+e.set_graph_steps(20)
+try:
+    e.step(20)
+except EngineError as err:
+    print("CHILD OK", err)
+"""
+
+
+def test_steps_run_plainly_where_no_graph_is_to_be_had(tmp_path):
+    """hipGraphInstantiate replaced by one that always fails: a graph that the
+    engine chose by itself is given up, one that the caller asked for is an error"""
+    src = tmp_path / "nograph.c"
+    src.write_text("int hipGraphInstantiate(void *e, void *g, void *n, char *b, unsigned long s)"
+                   "{ *(void **)e = 0; return 2; }\n")
+    lib = tmp_path / "nograph.so"
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(lib), str(src)], check=True)
+    r = subprocess.run([sys.executable, "-c", CHILD, str(lib)], capture_output=True, text=True,
+                       cwd=Path(__file__).resolve().parents[1], timeout=100)
+    assert r.returncode == 0 and "CHILD OK" in r.stdout, r.stdout + r.stderr
