@@ -430,6 +430,7 @@ size_t stage_bytes(size_t bytes) {
 
 // reference AoS (N x 3) -> device layout in device order
 void upload_vec(jh_ctx *c, const double *aos, double *dst, bool spin) {
+  HIPCHK(hipSetDevice(c->device));  // the calling thread may use another one
   const int64_t n = c->n;
   const size_t bytes = sizeof(double) * 3 * (size_t)n;
   const void *from = aos;
@@ -485,6 +486,7 @@ void copy_out(jh_ctx *c, const char *src, char *dst, size_t bytes) {
 
 // device layout -> reference AoS
 void download_vec(jh_ctx *c, const double *src, double *aos, bool spin) {
+  HIPCHK(hipSetDevice(c->device));  // its events are made on the current device
   const int64_t n = c->n;
   const size_t bytes = sizeof(double) * 3 * (size_t)n;
   const bool staged = c->stage.try_alloc(stage_bytes(bytes));

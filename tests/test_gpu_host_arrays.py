@@ -2,6 +2,10 @@
 bit for bit, at the sizes where the way of the copy changes (written to pinned
 memory by the kernel, one chunk, several chunks on several threads) and in
 both device orders."""
+import subprocess
+import sys
+from pathlib import Path
+
 import numpy as np
 import pytest
 
@@ -45,3 +49,38 @@ def test_basis_major_order_round_trip(engine_factory, L):
     assert np.array_equal(e.get_spins(), s)
     e.set_spins(-s)
     assert np.array_equal(e.get_spins(), -s)
+
+
+CHILD = """
+import ctypes, sys, threading
+shim = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)  # before the engine's own HIP library
+import numpy as np
+from jams_amd import configs
+from jams_amd.host import Simulation
+sim = Simulation(configs.sc_config(L=(40, 40, 40), temperature=10.0), device=0, output_dir="/tmp")
+e = sim.engine()
+e.step(1)
+s = e.get_spins()
+for call in (e.get_spins, lambda: e.set_spins(s), e.fields, lambda: e.get_noise(1),
+             lambda: e.set_noise(s)):
+    before = shim.calls()
+    t = threading.Thread(target=call)
+    t.start()
+    t.join()
+    assert shim.calls() > before
+print("CHILD OK")
+"""
+
+
+def test_transfers_bind_the_context_s_device(tmp_path):
+    """A thread whose current device is another one reads and sets arrays: each
+    transfer selects the context's device (counted by a hipSetDevice that
+    stands in for the library's; the one device is current anyway)."""
+    src = tmp_path / "device.c"
+    src.write_text("static int n; int hipSetDevice(int d) { __sync_fetch_and_add(&n, 1); return d != 0; }"
+                   " int calls(void) { return n; }\n")
+    lib = tmp_path / "device.so"
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(lib), str(src)], check=True)
+    r = subprocess.run([sys.executable, "-c", CHILD, str(lib)], capture_output=True, text=True,
+                       cwd=Path(__file__).resolve().parents[1], timeout=100)
+    assert r.returncode == 0 and "CHILD OK" in r.stdout, r.stdout + r.stderr
