@@ -152,18 +152,32 @@ __device__ __forceinline__ void xfield32(const XView &x, const float *__restrict
 // together, so a row of 6 waits for memory twice with U = 4 and a row of 14
 // four times (entry by entry after the full batches: 3 and 5 times).
 template <int U, class F>
-__device__ __forceinline__ void row_batches(int len, F &&f) {
-  int k = 1;
-  for (; k + U <= len + 1; k += U) f(k, std::integral_constant<int, U>{});
-  if constexpr (U > 1) {
-    const int rest = len + 1 - k;
-    if constexpr (U > 4)
-      if (rest & 4) { f(k, std::integral_constant<int, 4>{}); k += 4; }
-    if constexpr (U > 2)
-      if (rest & 2) { f(k, std::integral_constant<int, 2>{}); k += 2; }
-    if (rest & 1) f(k, std::integral_constant<int, 1>{});
+__host__ __device__ __forceinline__ constexpr void row_tail(int k, int rest, F &&f) {
+  if constexpr (U > 0) {
+    if (rest & U) {
+      f(k, std::integral_constant<int, U>{});
+      k += U;
+    }
+    row_tail<U / 2>(k, rest, f);
   }
 }
+template <int U, class F>
+__host__ __device__ __forceinline__ constexpr void row_batches(int len, F &&f) {
+  static_assert(U > 0 && (U & (U - 1)) == 0, "the tail is split by the bits of U - 1");
+  int k = 1;
+  for (; k + U <= len + 1; k += U) f(k, std::integral_constant<int, U>{});
+  row_tail<U / 2>(k, len + 1 - k, f);
+}
+// the entries that a row of `len` hands out in order (-1: one was skipped)
+template <int U>
+constexpr int row_entries(int len) {
+  int n = 0;
+  row_batches<U>(len, [&](int k, auto count) { n = n >= 0 && k == n + 1 ? n + count : -1; });
+  return n;
+}
+static_assert(row_entries<1>(3) == 3 && row_entries<4>(0) == 0 && row_entries<4>(7) == 7 &&
+                  row_entries<8>(15) == 15 && row_entries<16>(31) == 31 && row_entries<32>(95) == 95,
+              "every entry once, at any unroll");
 
 // exchange field of spin i from its row pattern (at word o), FP64, reference
 // order
