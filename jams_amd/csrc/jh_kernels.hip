@@ -1517,8 +1517,11 @@ __device__ __forceinline__ void ln_field(const LnView &ln, int sid, int xw, int 
 // 64^3 x 2, 11.9 instead of 11.2 at 32^2 x 64 x 2).  The predictors are the same
 // at 5, 6 and 8.  With two cells per lane a cap costs more than it gives (128^3 x
 // 2, FP32-field step 326 us without, 377 at 5 and 455 at 6 waves).
-template <int PHASE, int P>
-constexpr int kLnWaves = PHASE == 0 ? JH_LN_PRED_WAVES : P == 1 ? 6 : 1;
+// The general local terms (GEN: ac field, K2 or K3 anisotropy) take 160 VGPRs and
+// keep them: at 6 waves 72 to 130 are spilled (with K2, corrector at 64^3 x 2:
+// FP64 67.2 -> 97.9 us, FP32-field 37.4 -> 64.3).
+template <int PHASE, int P, bool GEN>
+constexpr int kLnWaves = PHASE == 0 ? JH_LN_PRED_WAVES : P == 1 && !GEN ? 6 : 1;
 // The corrector's own s, ds and noise: read before the field (FP32-field
 // form: it forms s* from them) or after it (FP64, fewer live registers)
 #ifndef JH_LN_EARLY64
@@ -1530,7 +1533,7 @@ constexpr bool kLnEarlyOwn = kEarlyOwn<PREC> || JH_LN_EARLY64;
 // constant 0 and its parameters are read through the scalar unit.
 template <int PREC, bool DIAG, int PHASE, bool GEN, int P, bool ONE>
 __global__ void __launch_bounds__(kLnBlock)
-__attribute__((amdgpu_waves_per_eu(kLnWaves<PHASE, P>))) k_heun_ln(const KParams p, const LnView ln) {
+__attribute__((amdgpu_waves_per_eu(kLnWaves<PHASE, P, GEN>))) k_heun_ln(const KParams p, const LnView ln) {
   const int rlb = ln.rlblocks;
   if ((int)blockIdx.x < rlb) {
     // FP64 row list: the rows whose z neighbours wrap, each summed in its own
