@@ -888,12 +888,14 @@ __device__ __forceinline__ bool grid_barrier(unsigned *sync, unsigned limit) {
 // grid holds at most as many workgroups as are resident at once; workgroup w
 // takes the spin blocks w, w + G, w + 2G, ... of the XCD-ordered numbering
 // (with G a multiple of 8 each XCD keeps a contiguous range, as in k_heun).
-// The tables are staged in LDS once for both phases.  The corrector reads the
-// FP32 copy the predictor wrote and writes the other (g32 and w32 swap).
+// The tables are staged in LDS once for both phases.  q: the corrector's
+// parameters, p but for the FP32 copies (it reads the one the predictor wrote
+// and writes the other).  Made in the kernel, that copy went to scratch, 400 to
+// 464 bytes per lane (256 replicas FP32-field: 835 us per step, so 666).
 template <int PREC, int XVk, bool GEN>
 __global__ void __launch_bounds__(kMaxBlock)
 __attribute__((amdgpu_waves_per_eu(kMinWaves<PREC, XVk>)))
-k_heun_step(const KParams p, unsigned *sync, unsigned limit) {
+k_heun_step(const KParams p, const KParams q, unsigned *sync, unsigned limit) {
   extern __shared__ __align__(16) unsigned char lds[];
   load_table<PREC, XVk>(p.x, lds);
   if constexpr (xv_typed(XVk)) __syncthreads();
@@ -907,9 +909,6 @@ k_heun_step(const KParams p, unsigned *sync, unsigned limit) {
     }
   }
   if (!grid_barrier(sync, limit)) return;
-  KParams q = p;
-  q.g32 = p.w32;
-  q.w32 = const_cast<float *>(p.g32);
   for (int64_t v = blockIdx.x; v < nv; v += gridDim.x) {
     const int64_t i = step_block(q, xcd_block(v, nv)) * blockDim.x + threadIdx.x;
     if (i < q.n) {
@@ -2011,7 +2010,10 @@ static hipError_t launch_heun_step_k(const KParams &p, int bs, int cus, unsigned
   const int64_t nv = (p.n + bs - 1) / bs;
   int64_t g = std::min<int64_t>(nv, (int64_t)per * cus);
   if (g >= 8) g -= g % 8;
-  hipLaunchKernelGGL(fn, dim3((unsigned)g), dim3(bs), lds, st, p, sync, limit);
+  KParams q = p;
+  q.g32 = p.w32;
+  q.w32 = const_cast<float *>(p.g32);
+  hipLaunchKernelGGL(fn, dim3((unsigned)g), dim3(bs), lds, st, p, q, sync, limit);
   return hipGetLastError();
 }
 

@@ -44,3 +44,10 @@ def test_no_spills(kernels, pattern):
     found = {n: k for n, k in kernels.items() if re.search(pattern, n)}
     assert found
     assert not {n: k for n, k in found.items() if k[1] or k[2]}
+
+
+def test_persistent_step_copies_no_parameters(kernels):
+    """its parameters are about 400 bytes; spilled scalars take less than 100"""
+    found = {n: k for n, k in kernels.items() if "k_heun_step<" in n}
+    assert found and all(k[1] == 0 for k in found.values())
+    assert not {n: k for n, k in found.items() if k[2] > 100}
