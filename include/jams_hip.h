@@ -276,7 +276,9 @@ int jh_phase_bytes(jh_ctx *ctx, int phase, double *fmt_bytes, double *csr_bytes)
  * stream (no host copy), and its algorithmic HBM bytes. */
 int jh_time_term(jh_ctx *ctx, int term, int reps, double *ms_per_eval);
 int jh_term_bytes(jh_ctx *ctx, int term, double *bytes);
-/* Text summary of the device formats chosen (for logs). */
+/* Text summary (for logs) of the device formats chosen and of what the next
+ * steps run as: launch=two, launch=persistent or launch=many (many steps in one
+ * launch of one workgroup), graph=<steps per replay, 0: none>. */
 int jh_describe(jh_ctx *ctx, char *buf, int64_t buflen);
 int jh_synchronize(jh_ctx *ctx);
 

@@ -2919,6 +2919,9 @@ int jh_describe(jh_ctx *c, char *buf, int64_t buflen) {
                                 "pattern-full-global", "pattern-uniform-diag",
                                 "pattern-uniform-full", "pattern-uniform-pairs-iso",
                                 "pattern-uniform-pairs-dmi"};
+    // what the next steps run as
+    const bool many = many_steps(c);
+    const int graph = many ? 0 : c->graph_steps > 0 ? c->graph_steps : auto_graph_steps(c);
     char tmp[512];
     std::snprintf(tmp, sizeof tmp,
                   "n=%lld prec=%s exchange=%s entries=%lld tensors=%d colbits=%d patterns=%d "
@@ -2929,7 +2932,7 @@ int jh_describe(jh_ctx *c, char *buf, int64_t buflen) {
                   (long long)c->nent, c->ntab > 0 ? c->ntab - 1 : 0, c->colbits,
                   c->npatterns, c->pat_words, c->pat_lds, (long long)c->nuniform,
                   (long long)c->nslices, (long long)c->npaired, c->order_nb, c->nclass,
-                  (int)c->terms.size(), c->noise_mode, c->launch_block(), c->nrep, c->graph_steps,
+                  (int)c->terms.size(), c->noise_mode, c->launch_block(), c->nrep, graph,
                   c->integrator == JH_INTEGRATOR_RK4 ? "rk4" : "heun");
     std::string out = tmp;
     if (c->st_on) {
@@ -2950,7 +2953,9 @@ int jh_describe(jh_ctx *c, char *buf, int64_t buflen) {
     }
     const int dip = dipole_term(c);
     if (dip >= 0) out += " " + c->dipoles[dip]->describe(c->prec == PR_FP32);
-    out += c->step_launch == JH_STEP_LAUNCH_PERSISTENT ? " launch=persistent" : " launch=two";
+    out += many                                          ? " launch=many"
+           : c->step_launch == JH_STEP_LAUNCH_PERSISTENT ? " launch=persistent"
+                                                         : " launch=two";
     if (buf && buflen > 0) {
       std::strncpy(buf, out.c_str(), (size_t)buflen - 1);
       buf[buflen - 1] = 0;

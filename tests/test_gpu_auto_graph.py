@@ -59,6 +59,22 @@ def test_replays_match_short_calls_bitwise(name):
         s.close()
 
 
+def test_describe_tells_the_graph():
+    sim = Simulation(CASES["heun"], device=0, output_dir="/tmp")
+    e = sim.engine()
+    assert "graph=0 " in e.describe()
+    e.step(499)
+    assert "graph=0 " in e.describe()
+    e.step(1)
+    assert "graph=20 " in e.describe()
+    e.set_graph_steps(7)
+    assert "graph=7 " in e.describe()
+    e.set_graph_steps(0)
+    e.step(600)
+    assert "graph=0 " in e.describe()
+    sim.close()
+
+
 CHILD = """
 import ctypes, sys
 ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)  # before the engine's own HIP library

@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 
 from jams_amd import configs
+from jams_amd.engine import STEP_LAUNCH_PERSISTENT, XFMT_BLOCK, XFMT_TYPED
 from jams_amd.host import Simulation
 from oracle import pyoracle as po
 from tests import systems as S
@@ -81,3 +82,54 @@ def test_odd_numbers_of_spins(L, precision):
                              precision=precision)
     for (a, _, ma), (b, _, mb) in zip(run(text, 0, (1, 60)), run(text, 128, (1, 60))):
         assert np.array_equal(a, b) and np.array_equal(ma, mb)
+
+
+@pytest.mark.parametrize("text,many", [
+    (configs.sc_config(L=(2, 1, 1), periodic=(False,) * 3, temperature=5.0), True),
+    (configs.sc_config(L=(3, 3, 7), temperature=10.0, precision="fp32-field"), True),
+    (configs.sc_config(L=(5, 13, 1), periodic=(False,) * 3, temperature=300.0), True),
+    (configs.sc_config(L=(8, 8, 16)), True),
+    (configs.sc_config(L=(9, 9, 12), periodic=(False,) * 3, temperature=20.0), True),
+    (configs.c2(8), True), (configs.c2(8, precision="fp32-field"), True),
+    # one spin more than a workgroup's threads; RK4; a dipole term; power-4 anisotropy
+    (configs.sc_config(L=(41, 25, 1), periodic=(False,) * 3), False),
+    (configs.c1(8).replace("llg-heun-gpu", "llg-rk4-gpu"), False),
+    (configs.sc_config(L=(5, 5, 3), periodic=(False,) * 3, dipole_rcut=3.0), False),
+    (configs.c2(8).replace('"K1"', '"K2"'), False)])
+def test_which_systems_take_the_launch(text, many):
+    """the comparisons above are between two launches, and this one says which"""
+    sim = Simulation(text, device=0, output_dir="/tmp")
+    e = sim.engine()
+    assert ("launch=many" in e.describe()) == many, e.describe()
+    e.set_block_size(256)
+    assert "launch=two" in e.describe()
+    e.set_block_size(0)
+    assert ("launch=many" in e.describe()) == many
+    if many:
+        e.set_step_launch(STEP_LAUNCH_PERSISTENT)
+        assert "launch=persistent" in e.describe()
+    sim.close()
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32-field"])
+@pytest.mark.parametrize("L", [(3, 3, 3), (5, 13, 1), (7, 10, 9), (8, 8, 16)])
+def test_typed_rows(L, precision):
+    """tensors by id per entry instead of row patterns, and BLOCK, which keeps two launches"""
+    text = configs.sc_config(L=L, periodic=(False,) * 3, temperature=20.0, seed=4,
+                             precision=precision)
+    got = []
+    for fmt, block in ((XFMT_TYPED, 0), (XFMT_TYPED, 256), (XFMT_BLOCK, 0)):
+        sim = Simulation(text, device=0, output_dir="/tmp")
+        e = sim.engine()
+        e.set_exchange_format(fmt)
+        e.set_block_size(block)
+        many = fmt == XFMT_TYPED and block == 0
+        assert ("launch=many" in e.describe()) == many, e.describe()
+        assert ("exchange=typed-diag" in e.describe()) == (fmt == XFMT_TYPED)
+        for n in (1, 2, 70):
+            e.step(n)
+        got.append(e.get_spins())
+        sim.close()
+    assert np.array_equal(got[0], got[1])
+    if precision == "fp64":
+        assert np.array_equal(got[0], got[2])
