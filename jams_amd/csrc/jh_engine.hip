@@ -381,7 +381,7 @@ struct jh_ctx {
   int graph_steps = 0;              // steps per captured graph (0: plain launches,
                                     // or the engine's own choice, auto_graph)
   bool auto_graph = true;
-  int64_t steps_run = 0;            // plain steps since the last layout
+  int64_t steps_run = 0;            // plain steps since the launches last changed
   hipGraph_t graph = nullptr;
   hipGraphExec_t gexec = nullptr;
   DevBuf<uint64_t> dstep;
@@ -393,6 +393,11 @@ struct jh_ctx {
     if (graph) (void)hipGraphDestroy(graph);
     gexec = nullptr;
     graph = nullptr;
+  }
+  // the steps' launches change: no graph of them until a run is long again
+  void new_launches() {
+    drop_graph();
+    steps_run = 0;
   }
 };
 
@@ -2461,10 +2466,13 @@ int jh_set_noise(jh_ctx *c, const double *w) {
   return guarded(c, [&] {
     require_sites(c);
     if (!w) JH_THROW(JH_ERR_INVALID, "jh_set_noise: null");
+    const double *held = c->noise_mode == NM_INJECTED ? c->winj.p : nullptr;
     c->winj.alloc((size_t)(3 * c->n));
     upload_vec(c, w, c->winj.p, false);
     c->noise_mode = NM_INJECTED;
-    c->drop_graph();  // its kernels hold the noise mode and buffer
+    // a graph's kernels hold the noise mode and buffer; new values in the same
+    // buffer leave it as it is (a caller may set them before every few steps)
+    if (c->winj.p != held) c->new_launches();
   });
 }
 
@@ -2804,8 +2812,8 @@ int jh_set_block_size(jh_ctx *c, int threads) {
     if (threads != 0 && (threads < 64 || threads > kStMaxBlock || threads % 64 != 0))
       JH_THROW(JH_ERR_INVALID, "workgroup size must be 0 or a multiple of 64 in [64, 1024]");
     if (threads != c->block && (c->st_on || c->have_lattice)) c->dirty = true;  // tile shape
+    if (threads != c->block) c->new_launches();
     c->block = threads;
-    c->drop_graph();
   });
 }
 

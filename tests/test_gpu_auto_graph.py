@@ -75,6 +75,34 @@ def test_describe_tells_the_graph():
     sim.close()
 
 
+@pytest.mark.parametrize("chosen", [0, 20])
+def test_noise_set_before_every_few_steps(chosen):
+    """New values in the same buffer keep the graph, the engine's own and the
+    caller's; only the first ones, or another workgroup size, end it."""
+    a, b = (Simulation(CASES["heun"], device=0, output_dir="/tmp") for _ in range(2))
+    e, f = a.engine(), b.engine()
+    if chosen:
+        e.set_graph_steps(chosen)
+    e.step(600)
+    f.set_graph_steps(0)
+    f.step(600)
+    rng = np.random.default_rng(8)
+    for k in range(40):
+        w = rng.standard_normal((e.n, 3))
+        for q in (e, f):
+            q.set_noise(w)
+            q.step(20)
+        assert (f"graph={20 if chosen or k > 24 else 0} " in e.describe()) or k == 24, k
+    assert np.array_equal(e.get_spins(), f.get_spins())
+    e.set_block_size(128)
+    assert f"graph={chosen} " in e.describe()
+    for q in (e, f):
+        q.step(100)
+    assert np.array_equal(e.get_spins(), f.get_spins())
+    a.close()
+    b.close()
+
+
 CHILD = """
 import ctypes, sys
 ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)  # before the engine's own HIP library
