@@ -421,7 +421,8 @@ inline int64_t dev_of(const jh_ctx *c, int64_t i) {
 // with kStageSlots chunks of the pinned memory of its own, so that the page
 // faults are spread and overlap the transfers.  At most kStageBytes is pinned
 // per context.  Arrays of kDirectBytes or less are written into the pinned
-// memory by the layout kernel itself (a copy command costs 10 us).
+// memory, or read from it, by the layout kernel itself (a copy command costs 10
+// us).
 constexpr size_t kStageChunk = 1 << 20;
 constexpr int kStageSlots = 2, kStageThreads = 8;
 constexpr size_t kStageBytes = kStageChunk * kStageSlots * kStageThreads;
@@ -438,15 +439,20 @@ void upload_vec(jh_ctx *c, const double *aos, double *dst, bool spin) {
   HIPCHK(hipSetDevice(c->device));  // the calling thread may use another one
   const int64_t n = c->n;
   const size_t bytes = sizeof(double) * 3 * (size_t)n;
-  const void *from = aos;
+  const double *from = aos;
   // up to a chunk through pinned memory: the runtime pins the pages of a
   // pageable source for the transfer, 0.3 ms at 0.8 MB against 0.08
-  if (bytes <= kStageChunk && c->stage.try_alloc(stage_bytes(bytes))) {
+  const bool staged = bytes <= kStageChunk && c->stage.try_alloc(stage_bytes(bytes));
+  if (staged) {
     std::memcpy(c->stage.p, aos, bytes);
-    from = c->stage.p;
+    from = reinterpret_cast<const double *>(c->stage.p);
   }
-  HIPCHK(hipMemcpyAsync(c->aos.p, from, bytes, hipMemcpyHostToDevice, c->stream));
-  HIPCHK(launch_vec_layout(c->aos.p, dst, n, c->order_nb, c->order_cells, spin, false, c->stream));
+  // small ones are read from there by the layout kernel itself
+  if (!staged || bytes > kDirectBytes) {
+    HIPCHK(hipMemcpyAsync(c->aos.p, from, bytes, hipMemcpyHostToDevice, c->stream));
+    from = c->aos.p;
+  }
+  HIPCHK(launch_vec_layout(from, dst, n, c->order_nb, c->order_cells, spin, false, c->stream));
   HIPCHK(hipStreamSynchronize(c->stream));
 }
 
