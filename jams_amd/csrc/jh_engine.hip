@@ -276,7 +276,6 @@ struct jh_ctx {
   DevBuf<double> sq;        // RK4: second stage-input buffer (stages alternate sp, sq)
   DevBuf<float> sq32;
   DevBuf<double> red_partial;
-  DevBuf<double> aos;            // a vector array in the host layout
   // pinned host memory: the reductions' results (kernels write them there) and
   // the staging of arrays read back, with one event per kStageChunk of it
   PinnedBuf<double> hres;
@@ -434,6 +433,13 @@ size_t stage_bytes(size_t bytes) {
   return std::min(kStageBytes, (bytes + kStageChunk - 1) / kStageChunk * kStageChunk);
 }
 
+// A device array of 3N doubles for a vector array in the host layout, beside
+// the array that is read or written: the fields' output, which holds nothing
+// from one call to the next, or ds, which every step writes before it reads.
+double *spare_array(jh_ctx *c, const double *other) {
+  return other == c->fout.p ? c->ds.p : c->fout.p;
+}
+
 // reference AoS (N x 3) -> device layout in device order
 void upload_vec(jh_ctx *c, const double *aos, double *dst, bool spin) {
   HIPCHK(hipSetDevice(c->device));  // the calling thread may use another one
@@ -449,8 +455,9 @@ void upload_vec(jh_ctx *c, const double *aos, double *dst, bool spin) {
   }
   // small ones are read from there by the layout kernel itself
   if (!staged || bytes > kDirectBytes) {
-    HIPCHK(hipMemcpyAsync(c->aos.p, from, bytes, hipMemcpyHostToDevice, c->stream));
-    from = c->aos.p;
+    double *tmp = spare_array(c, dst);
+    HIPCHK(hipMemcpyAsync(tmp, from, bytes, hipMemcpyHostToDevice, c->stream));
+    from = tmp;
   }
   HIPCHK(launch_vec_layout(from, dst, n, c->order_nb, c->order_cells, spin, false, c->stream));
   HIPCHK(hipStreamSynchronize(c->stream));
@@ -502,15 +509,15 @@ void download_vec(jh_ctx *c, const double *src, double *aos, bool spin) {
   const size_t bytes = sizeof(double) * 3 * (size_t)n;
   const bool staged = c->stage.try_alloc(stage_bytes(bytes));
   const bool direct = staged && bytes <= kDirectBytes;
-  HIPCHK(launch_vec_layout(src, direct ? reinterpret_cast<double *>(c->stage.p) : c->aos.p, n,
-                           c->order_nb, c->order_cells, spin, true, c->stream));
+  double *tmp = direct ? reinterpret_cast<double *>(c->stage.p) : spare_array(c, src);
+  HIPCHK(launch_vec_layout(src, tmp, n, c->order_nb, c->order_cells, spin, true, c->stream));
   if (direct) {
     HIPCHK(hipStreamSynchronize(c->stream));
     std::memcpy(aos, c->stage.p, bytes);
     return;
   }
   if (!staged) {  // no pinned memory to be had
-    HIPCHK(hipMemcpyAsync(aos, c->aos.p, bytes, hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(hipMemcpyAsync(aos, tmp, bytes, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     return;
   }
@@ -519,7 +526,7 @@ void download_vec(jh_ctx *c, const double *src, double *aos, bool spin) {
     HIPCHK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
     c->stage_ev.push_back(ev);
   }
-  copy_out(c, reinterpret_cast<const char *>(c->aos.p), reinterpret_cast<char *>(aos), bytes);
+  copy_out(c, reinterpret_cast<const char *>(tmp), reinterpret_cast<char *>(aos), bytes);
 }
 
 // ---- exchange input conversion -------------------------------------------
@@ -2286,7 +2293,6 @@ int jh_set_sites(jh_ctx *c, int64_t n, const double *mus, const double *gyro, co
     c->fout.alloc((size_t)(3 * n));
     const int64_t nb = (n + kBlock - 1) / kBlock;
     c->red_partial.alloc((size_t)(4 * nb));
-    c->aos.alloc((size_t)(3 * n));
     c->hres.alloc(4);
     // pinned here, once: the first array read back does not wait for it
     (void)c->stage.try_alloc(stage_bytes(sizeof(double) * 3 * (size_t)n));

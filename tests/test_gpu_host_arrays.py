@@ -2,6 +2,7 @@
 bit for bit, at the sizes where the way of the copy changes (written to pinned
 memory by the kernel, one chunk, several chunks on several threads) and in
 both device orders."""
+import ctypes
 import subprocess
 import sys
 from pathlib import Path
@@ -49,6 +50,47 @@ def test_basis_major_order_round_trip(engine_factory, L):
     assert np.array_equal(e.get_spins(), s)
     e.set_spins(-s)
     assert np.array_equal(e.get_spins(), -s)
+
+
+def test_no_device_memory_for_the_transfers(engine_factory):
+    """s, s*, ds and the field output: four arrays of 24 bytes per spin, and the
+    transfers take no fifth one"""
+    def free_bytes():
+        free, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        return free.value
+
+    n = 1 << 22
+    e = engine_factory()
+    hip = e.lib  # the engine's own HIP library is found through it
+    before = free_bytes()
+    e.set_sites(np.ones(n), np.ones(n), np.full(n, 0.1))
+    s = np.random.default_rng(3).standard_normal((n, 3))
+    e.set_spins(s)
+    assert np.array_equal(e.get_spins(), s)
+    assert before - free_bytes() <= 4 * 24 * n + (16 << 20)
+
+
+def test_reads_between_steps_leave_them_alone(engine_factory):
+    """spins, fields and noise read back between steps of both integrators, and
+    the steps that follow, against a context that is not read"""
+    for integrator in (0, 1):
+        b = S.c2(24)
+        got = []
+        for reads in (True, False):
+            e = b.engine(engine_factory)
+            e.set_integrator(integrator)
+            e.set_thermostat(300.0, 7)
+            for _ in range(3):
+                e.step(2)
+                if reads:
+                    s = e.get_spins()
+                    h = e.fields()
+                    w = e.get_noise(1)
+                    assert np.array_equal(h, e.fields()) and np.array_equal(w, e.get_noise(1))
+                    assert np.array_equal(s, e.get_spins())
+            got.append(e.get_spins())
+        assert np.array_equal(*got)
 
 
 CHILD = """
