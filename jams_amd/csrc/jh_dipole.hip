@@ -91,22 +91,20 @@ std::vector<int> factorise(int n) {
 }
 
 // Radices of an axis of the fused kernels: the fewest of those they are built
-// for (then the smallest), since every stage costs two barriers and a trip
-// through LDS: 180 = 15 x 12, 150 = 15 x 10, 400 = 10 x 10 x 4 against 4 x 5 x
-// 3 x 3, 2 x 5 x 5 x 3 and 8 x 2 x 5 x 5.  512 stays 8 x 8 x 8, which has
-// stages of its own.  Empty when n has a prime factor above 7.
-std::vector<int> fused_radices(int n) {
+// for (then those of the smallest sum), since every stage costs two barriers
+// and a trip through LDS: 180 = 15 x 12, 150 = 15 x 10, 400 = 10 x 8 x 5
+// against 4 x 5 x 3 x 3, 2 x 5 x 5 x 3 and 8 x 2 x 5 x 5.  512 stays 8 x 8 x
+// 8, which has stages of its own; 1 has none.  False when n has a prime factor
+// above 7.
+bool fused_radices(int n, std::vector<int> &best) {
   static const int set[] = {16, 15, 12, 10, 9, 8, 7, 6, 5, 4, 3, 2};
-  std::vector<int> best;
+  best.clear();
+  if (n == 1) return true;
   int best_sum = 0;
   for (int r : set) {
-    if (n % r) continue;
-    std::vector<int> s{r};
-    if (n > r) {
-      const std::vector<int> rest = fused_radices(n / r);
-      if (rest.empty()) continue;
-      s.insert(s.end(), rest.begin(), rest.end());
-    }
+    std::vector<int> s;
+    if (n % r || !fused_radices(n / r, s)) continue;
+    s.insert(s.begin(), r);
     int sum = 0;
     for (int q : s) sum += q;
     if (best.empty() || s.size() < best.size() || (s.size() == best.size() && sum < best_sum)) {
@@ -114,7 +112,7 @@ std::vector<int> fused_radices(int n) {
       best_sum = sum;
     }
   }
-  return best;
+  return !best.empty();
 }
 
 // exp(-2 pi i t / n), t < n.  Entries of the first half are evaluated in long
@@ -1012,7 +1010,8 @@ class DipoleFFTImpl : public DipoleFFT {
   int64_t n, Q2, M;  // M = P0 P1 Q2
   bool real_tensor = false;  // W(n) = W(-n): the transformed tensor is real
   std::vector<int> rad[3];   // the separate passes' radices
-  std::vector<int> frad[3];  // the fused kernels' (empty: not for them)
+  std::vector<int> frad[3];  // the fused kernels'
+  bool fok[3];               // whether they have the length
   DBuf<double> mus;
   Plane<double> f64;
   Plane<float> f32;
@@ -1074,7 +1073,7 @@ class DipoleFFTImpl : public DipoleFFT {
   // the grid would otherwise leave compute units idle
   template <class T>
   int fused_lines() const {
-    if (nb != 1 || !real_tensor || frad[0].empty()) return 0;
+    if (nb != 1 || !real_tensor || !fok[0]) return 0;
     const size_t c = sizeof(typename fft::C2<T>::type);
     int fit = 0;
     for (int by = 8; by >= 1; by /= 2) {
@@ -1232,7 +1231,7 @@ class DipoleFFTImpl : public DipoleFFT {
   // than 5 or 2)
   template <class T>
   int zy_split() const {
-    if (!direct_z() || frad[1].empty()) return 0;
+    if (!direct_z() || !fok[1]) return 0;
     for (int ns = Q2 >= 4 ? JH_ZY_SPLIT : 1; ns <= Q2; ++ns) {
       const int lw = (int)((Q2 + ns - 1) / ns);
       if (zy_lds<T>(lw) <= kMaxPassLds && zy_threads<T>(lw) <= 512) return ns;
@@ -1504,7 +1503,8 @@ DipoleFFT *DipoleFFT::create(const int32_t size[3], const int32_t periodic[3], i
     if (pass_lds<double>(d->P[a], 1, true) > kMaxPassLds)
       return fail("padded dimension too long for one workgroup's LDS (at most 2048)");
     d->rad[a] = factorise(d->P[a]);
-    d->frad[a] = d->P[a] == 512 ? d->rad[a] : fused_radices(d->P[a]);
+    d->fok[a] = fused_radices(d->P[a], d->frad[a]);
+    if (d->P[a] == 512) d->frad[a] = d->rad[a];
     if ((int)d->rad[a].size() > fft::kMaxStages) return fail("too many FFT stages");
     for (int r : d->rad[a])
       if (r > 64) return fail("padded dimension has a prime factor above 64");
