@@ -257,9 +257,12 @@ int jh_set_step_launch(jh_ctx *ctx, int mode);
 /* Time `steps` steps of every exchange format that fits (PATTERN, TYPED,
  * BLOCK, and on a lattice STENCIL and LINE) at 128, 256 and 512 threads per
  * workgroup (STENCIL also 1024, LINE its one shape), each gathering format
- * also as one persistent launch per step, from the current state; keep the
- * fastest, restore the state; report (may be NULL) gets one line per
- * candidate and a last "chosen ..." line. */
+ * also as one persistent launch per step and, in a context that can, as many
+ * steps in one launch of one workgroup (block=0 launch=many), from the current
+ * state; keep the fastest, restore the state; report (may be NULL) gets one
+ * line per candidate and a last "chosen ..." line.  Two launches per step are
+ * timed in the graph that a context of this size replays by itself, where
+ * `steps` is long enough for it. */
 int jh_autotune(jh_ctx *ctx, int steps, char *report, int64_t len);
 
 /* ---- measurement -------------------------------------------------------- */

@@ -2108,6 +2108,18 @@ void build_graph(jh_ctx *c, int steps) {
   HIPCHK(hipGraphInstantiate(&c->gexec, c->graph, nullptr, nullptr, 0));
 }
 
+// build_graph for a graph that nobody asked for: false where it cannot be had
+bool try_graph(jh_ctx *c, int steps) {
+  try {
+    build_graph(c, steps);
+    return true;
+  } catch (const JhError &) {
+    c->drop_graph();
+    (void)hipGetLastError();
+    return false;
+  }
+}
+
 // Whether the context's steps run as many steps per launch of one workgroup
 // (k_heun_many).
 bool many_steps(const jh_ctx *c) {
@@ -2146,14 +2158,10 @@ void do_steps(jh_ctx *c, int64_t nsteps) {
   }
   int graph_steps = c->graph_steps > 0 ? c->graph_steps : auto_graph_steps(c);
   if (graph_steps > 0 && nsteps >= graph_steps && !c->gexec) {
-    try {
+    if (c->graph_steps > 0) {
       build_graph(c, graph_steps);
-    } catch (const JhError &) {
-      if (c->graph_steps > 0) throw;
-      // nobody asked for this graph: plain launches from here on
-      c->drop_graph();
-      (void)hipGetLastError();
-      c->auto_graph = false;
+    } else if (!try_graph(c, graph_steps)) {
+      c->auto_graph = false;  // plain launches from here on
       graph_steps = 0;
     }
   }
@@ -2848,6 +2856,9 @@ int jh_autotune(jh_ctx *c, int steps, char *report, int64_t len) {
     std::string rep;
     double best = 1e300;
     int best_fmt = fmt0, best_bs = bs0, best_sl = sl0;
+    bool best_many = false;
+    // the graph that two launches per step get by themselves in runs this long
+    const int replay = ag0 && c->n <= kAutoGraphSpins && steps >= kAutoGraphSteps ? kAutoGraphSteps : 0;
     for (int fmt : {JH_XFMT_PATTERN, JH_XFMT_TYPED, JH_XFMT_BLOCK, JH_XFMT_STENCIL, JH_XFMT_LINE}) {
       if (c->xh.empty() && fmt != JH_XFMT_PATTERN) continue;
       const bool stencil = fmt == JH_XFMT_STENCIL;
@@ -2862,10 +2873,14 @@ int jh_autotune(jh_ctx *c, int steps, char *report, int64_t len) {
           continue;  // this format does not fit the system
         }
       }
-      for (int bs : {128, 256, 512, 1024}) {
+      for (int bs : {0, 128, 256, 512, 1024}) {
+        if (bs == 0 && (stencil || line)) continue;
         if (bs == 1024 && !stencil) continue;
         if (line && bs != kLnBlock) continue;  // one shape: a wave per line
         c->block = bs;
+        // no size of its own: many steps in one launch, where they fit
+        const bool many = many_steps(c);
+        if (bs == 0 && !many) continue;
         if (stencil) {
           // the block size is the tile shape: lay it out again
           c->dirty = true;
@@ -2876,16 +2891,20 @@ int jh_autotune(jh_ctx *c, int steps, char *report, int64_t len) {
           }
         }
         // the gathering formats also as one persistent launch per step
-        const bool persist = persistent_unfit(c) == nullptr;
+        const bool persist = persistent_unfit(c) == nullptr && !many;
         for (int sl : {JH_STEP_LAUNCH_TWO, JH_STEP_LAUNCH_PERSISTENT}) {
           if (sl == JH_STEP_LAUNCH_PERSISTENT && !persist) continue;
           c->step_launch = sl;
           if (sl == JH_STEP_LAUNCH_PERSISTENT) ensure_step_sync(c);
+          c->drop_graph();
+          c->graph_steps = 0;
+          if (sl == JH_STEP_LAUNCH_TWO && !many && replay && try_graph(c, replay))
+            c->graph_steps = replay;
           HIPCHK(hipMemcpyAsync(c->s.p, save.p, sizeof(double) * 3 * c->n, hipMemcpyDeviceToDevice, c->stream));
           sync_f32(c);
           c->iteration = it0;
           c->time = t0;
-          do_steps(c, 2);
+          do_steps(c, std::max(2, c->graph_steps));
           HIPCHK(hipEventRecord(c->ev0, c->stream));
           do_steps(c, steps);
           HIPCHK(hipEventRecord(c->ev1, c->stream));
@@ -2896,13 +2915,14 @@ int jh_autotune(jh_ctx *c, int steps, char *report, int64_t len) {
           const double ms = (double)f / steps;
           char line[128];
           std::snprintf(line, sizeof line, "format=%d block=%d launch=%s %.4f ms/step\n", fmt, bs,
-                        sl == JH_STEP_LAUNCH_PERSISTENT ? "persistent" : "two", ms);
+                        many ? "many" : sl == JH_STEP_LAUNCH_PERSISTENT ? "persistent" : "two", ms);
           rep += line;
           if (ms < best) {
             best = ms;
             best_fmt = fmt;
             best_bs = bs;
             best_sl = sl;
+            best_many = many;
           }
         }
         c->step_launch = JH_STEP_LAUNCH_TWO;
@@ -2922,7 +2942,7 @@ int jh_autotune(jh_ctx *c, int steps, char *report, int64_t len) {
     c->time = t0;
     char line[128];
     std::snprintf(line, sizeof line, "chosen format=%d block=%d launch=%s", best_fmt, best_bs,
-                  best_sl == JH_STEP_LAUNCH_PERSISTENT ? "persistent" : "two");
+                  best_many ? "many" : best_sl == JH_STEP_LAUNCH_PERSISTENT ? "persistent" : "two");
     rep += line;
     if (report && len > 0) {
       std::strncpy(report, rep.c_str(), (size_t)len - 1);

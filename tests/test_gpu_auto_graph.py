@@ -118,6 +118,7 @@ for s, most in ((a, 19), (b, 700)):
         n -= most
 assert np.array_equal(a.engine().get_spins(), b.engine().get_spins())
 e = a.engine()
+print(b.engine().autotune(40))
 e.set_graph_steps(20)
 try:
     e.step(20)

@@ -122,6 +122,52 @@ def test_autotuned_launch_shape_gives_the_same_bits():
     tuned.close()
 
 
+@pytest.mark.parametrize("text", [
+    configs.c1(8), configs.c1(8, temperature=10.0, precision="fp32-field"), configs.c2(6)])
+def test_autotune_keeps_the_many_step_launch_of_a_small_system(text):
+    """a third of the time of two launches per step, so the fastest candidate"""
+    ref, tuned = (Simulation(text, device=0, output_dir="/tmp") for _ in range(2))
+    a, b = ref.engine(), tuned.engine()
+    report = b.autotune(40)
+    print(report)
+    assert report.splitlines()[-1].endswith("block=0 launch=many"), report
+    assert "launch=two" in report and "launch=persistent" in report
+    assert "launch=many" in b.describe()
+    assert b.iteration() == a.iteration()
+    for n in (3, 40):
+        a.step(n)
+        b.step(n)
+        if "fp64" in text:  # (the formats sum the FP32 form's terms in other orders)
+            assert np.array_equal(a.get_spins(), b.get_spins())
+        else:
+            assert np.abs(a.get_spins() - b.get_spins()).max() < 1e-4
+    ref.close()
+    tuned.close()
+
+
+@pytest.mark.parametrize("steps", [5, 40])
+def test_autotune_leaves_the_graph_to_come(steps):
+    """too many spins for one workgroup: two launches, timed in 20-step replays
+    where the caller's steps are as many, and replayed after 500 plain steps"""
+    ref, tuned = (Simulation(configs.c1(16, temperature=10.0), device=0, output_dir="/tmp")
+                  for _ in range(2))
+    a, b = ref.engine(), tuned.engine()
+    a.set_graph_steps(0)
+    report = b.autotune(steps)
+    assert "launch=many" not in report
+    if "launch=two" in report.splitlines()[-1]:
+        assert "graph=0 " in b.describe()
+        b.step(500)
+        a.step(500)
+        assert "graph=20 " in b.describe()
+    a.step(100)
+    b.step(100)
+    assert a.iteration() == b.iteration()
+    assert np.array_equal(a.get_spins(), b.get_spins())
+    ref.close()
+    tuned.close()
+
+
 @pytest.mark.parametrize("bs", [64, 128, 512])
 def test_block_sizes_give_the_same_bits(engine_factory, bs):
     from tests import systems as S
