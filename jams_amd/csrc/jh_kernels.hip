@@ -226,6 +226,7 @@ __device__ __forceinline__ void pfield64(const XView &x, const double *__restric
       for (int u = 0; u < C; ++u) accum(w[u] & tmask, v[u].x, v[u].y, z[u]);
     });
   } else {
+#pragma unroll kUnrollFor<XVk>
     for (int k = 1; k <= len; ++k) {
       const uint32_t w = pat[o + k];
       const int64_t j = i + (int64_t)(((int32_t)w) >> x.tbits);
