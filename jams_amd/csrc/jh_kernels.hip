@@ -1673,9 +1673,19 @@ __attribute__((amdgpu_waves_per_eu(kLnWaves<PHASE, P, GEN>))) k_heun_ln(const KP
 //   multiplies by CUDA's rsqrt; here 1 / sqrt, each correctly rounded).
 // ONE: no class table, the class is the constant 0 (its parameters then
 // come through the scalar unit).
+// FP64 rows of full tensors: with eight gathers in flight a stage takes 84 VGPRs,
+// five waves per SIMD; 78 fit six without a spill.  Five shells, step: 64^3 x 2
+// 198.4 -> 191.8 us (195.3 with the gathers not batched, 47 VGPRs), 128^3 x 2
+// 1536 -> 1457 (1540), 48^3 x 2 105.5 -> 105.4 (116.3).  At seven waves 5 spill:
+// 197, 1545, 111.7.  The FP32-field forms spill at six and keep what they take
+// (uniform full rows, 86: 64^3 x 2 120.4 us where not batched 134.5, 128^3 x 2
+// 1015 where 993).
+template <int PREC, int XVk, bool GEN>
+constexpr int kRk4Waves =
+    PREC == PR_FP64 && XVk == XV_PFULL && !GEN ? 6 : kMinWaves<PREC, XVk>;
 template <int PREC, int XVk, bool GEN, bool ONE>
 __global__ void __launch_bounds__(kMaxBlock)
-__attribute__((amdgpu_waves_per_eu(kMinWaves<PREC, XVk>))) k_rk4(const KParams p) {
+__attribute__((amdgpu_waves_per_eu(kRk4Waves<PREC, XVk, GEN>))) k_rk4(const KParams p) {
   extern __shared__ __align__(16) unsigned char lds[];
   const int64_t blk = xcd_block(blockIdx.x, gridDim.x);
   const int64_t i = blk * blockDim.x + threadIdx.x;

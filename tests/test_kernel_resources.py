@@ -51,3 +51,9 @@ def test_persistent_step_copies_no_parameters(kernels):
     found = {n: k for n, k in kernels.items() if "k_heun_step<" in n}
     assert found and all(k[1] == 0 for k in found.values())
     assert not {n: k for n, k in found.items() if k[2] > 100}
+
+
+def test_rk4_stages_of_full_tensors_leave_room_for_six_waves(kernels):
+    """<FP64, rows of full tensors by pattern, no general terms, ...>: 512 / 6 VGPRs"""
+    found = {n: k for n, k in kernels.items() if "k_rk4<0, 6, false, " in n}
+    assert len(found) == 2 and all(k[0] <= 80 for k in found.values())
