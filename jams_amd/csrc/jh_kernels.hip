@@ -33,9 +33,14 @@ namespace jh {
 constexpr int kGatherUnroll = JH_GATHER_UNROLL;
 // Tensor-table rows are indexed with 24-bit multiplies (__mul24, full rate;
 // a 32-bit multiply is a quarter-rate instruction): table ids are < 2^24.
-// full-tensor rows (9 products per neighbour) gain from more loads in flight
+// Full-tensor rows (9 products per neighbour) gain from more loads in flight,
+// except where they are what a pair program leaves over: eight of them took the
+// registers of the pairs (87 VGPRs in the predictor, 123 in the corrector; 70
+// and 94 with four), and bcc 128^3 x 2 with five shells gathered in the
+// FP32-field form took 407 us per step, 70 x 61 x 66 67.2, 36 x 33 x 35 20.4;
+// with four 386, 64.1 and 20.3.
 template <int XVk>
-constexpr int kUnrollFor = xv_diag(XVk) ? kGatherUnroll : 2 * kGatherUnroll;
+constexpr int kUnrollFor = xv_diag(XVk) || xv_pair(XVk) ? kGatherUnroll : 2 * kGatherUnroll;
 
 // FP32 gather copy of the spins: kG32 floats per spin, (x, y, z[, 0])
 __device__ __forceinline__ void load_g32(const float *__restrict__ src, uint32_t j, double &x,

@@ -53,7 +53,12 @@ def test_persistent_step_copies_no_parameters(kernels):
     assert not {n: k for n, k in found.items() if k[2] > 100}
 
 
-def test_rk4_stages_of_full_tensors_leave_room_for_six_waves(kernels):
-    """<FP64, rows of full tensors by pattern, no general terms, ...>: 512 / 6 VGPRs"""
-    found = {n: k for n, k in kernels.items() if "k_rk4<0, 6, false, " in n}
-    assert len(found) == 2 and all(k[0] <= 80 for k in found.values())
+@pytest.mark.parametrize("pattern,most", [
+    # <FP64, rows of full tensors by pattern, no general terms, ...>: six waves
+    (r"k_rk4<0, 6, false, ", 80),
+    # <FP32 field, pair programs with DMI, phase, no general terms, one class>:
+    # seven and five waves
+    (r"k_heun<1, 12, 0, false, 2>", 72), (r"k_heun<1, 12, 1, false, 2>", 96)])
+def test_full_tensors_leave_room_for_other_waves(kernels, pattern, most):
+    found = {n: k for n, k in kernels.items() if re.search(pattern, n)}
+    assert found and all(k[0] <= most for k in found.values())
