@@ -1532,9 +1532,10 @@ void prepare_exchange(jh_ctx *c) {
   // texture-address time it saves); jh_autotune times it beside the others
   const bool want_stencil = fmt == JH_XFMT_STENCIL;
   // AUTO takes LINE for a lattice whose rows hold at least kLnAutoMinRow
-  // neighbours: measured at bcc 128^3 x 2 with 58 neighbours it runs the
-  // step 1.25x (FP64) and 1.15x (FP32 form) faster than the gathers, at
-  // bcc 64^3 x 2 with 14 it runs 13 % and 5 % slower
+  // neighbours.  Step with LINE against the gathers, bcc 128^3 x 2 with 58
+  // neighbours: FP64 540 against 713 us, FP32 form 324 against 386; with 14:
+  // 64^3 x 2 46.0 against 35.7 and 38.1 against 33.4, 128^3 x 2 279 against 265
+  // and 224 against 225, 16^2 x 64 x 2 22.3 against 12.4 and 14.0 against 12.9
   const bool want_line = fmt == JH_XFMT_LINE ||
                          (fmt == JH_XFMT_AUTO && c->have_lattice && c->nrep == 0 &&
                           c->integrator == JH_INTEGRATOR_HEUN &&

@@ -353,9 +353,14 @@ __device__ __forceinline__ void stage_fixed(const Pass<T> &p, const typename C2<
   }
 }
 
-// Butterflies per thread of an in-place stage: R * kBF <= 8 complex values
-// in registers (with 16, the 512-thread workgroups hold 108-188 VGPRs and one
-// fits per CU; with 8, two do, and the passes run 25-30 % faster).
+// Butterflies per thread of an in-place stage.  Up to radix 8, R * kBF <= 8
+// complex values in registers (with 16, the 512-thread workgroups hold 108-188
+// VGPRs and one fits per CU; with 8, two do, and the passes run 25-30 %
+// faster).  The fused kernels' radices 9 to 16 are one butterfly, 9 to 16
+// values: k_dip_x_fused<double, 0> takes 107 VGPRs, four waves per SIMD instead
+// of five, the FP64 k_dip_zy_inv three or four, and the stages they save are
+// worth more (dipole evaluation in FP64, film 240 x 240 x 8 184 -> 144 us, 216
+// x 225 x 6 151 -> 132, 135 x 125 x 6 63.1 -> 61.3).
 constexpr int kbf_of(int R) { return R <= 8 ? 8 / R : 1; }
 template <class T, int R>
 constexpr int kBF = kbf_of(R);
