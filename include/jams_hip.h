@@ -230,7 +230,9 @@ int jh_reduce_magnetisation_replicas(jh_ctx *ctx, double *out);
 /* Run jh_step as replays of one captured hipGraph of `steps` Heun steps
  * (whatever is left over runs as plain launches); 0 disables graphs.  Without
  * a call, contexts of up to 2^18 spins replay a 20-step graph of their own
- * once they have run 500 steps, with the same results. */
+ * once they have run 500 steps, with the same results, and plain launches
+ * where that graph cannot be built.  A context that runs many steps per launch
+ * (jh_set_block_size) goes on doing so. */
 int jh_set_graph_steps(jh_ctx *ctx, int steps);
 /* Threads per workgroup of the step kernels: 64 .. 512, a multiple of 64;
  * 0 (the default) picks 256 or 512 by exchange format, and lets a context of
