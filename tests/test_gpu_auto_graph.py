@@ -3,6 +3,7 @@ plain steps: the same bits as calls too short for a replay, replay after
 replay, with reductions, field evaluations and set-up changes in between."""
 import subprocess
 import sys
+from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
 import numpy as np
@@ -101,6 +102,36 @@ def test_noise_set_before_every_few_steps(chosen):
     assert np.array_equal(e.get_spins(), f.get_spins())
     a.close()
     b.close()
+
+
+def test_contexts_on_several_threads():
+    """Each thread sets contexts up, steps them past the point where they capture
+    a graph and reads them, while the others do the same: the bits of the same
+    runs one after the other."""
+    texts = [configs.sc_config(L=(13, 11, 12), temperature=20.0, seed=3),
+             configs.sc_config(L=(13, 11, 12), temperature=20.0, seed=4, precision=F32),
+             configs.bcc_config(L=9, seed=5), CASES["film"]]
+
+    def go(text):
+        out = []
+        for _ in range(3):
+            s = Simulation(text, device=0, output_dir="/tmp")
+            e = s.engine()
+            for n in (490, 30, 75):
+                e.step(n)
+                out.append(e.get_spins())
+            e.set_thermostat(5.0, 9)
+            e.step(560)
+            out.append(e.get_spins())
+            out.append(e.magnetisation())
+            s.close()
+        return out
+
+    alone = [go(t) for t in texts]
+    with ThreadPoolExecutor(len(texts)) as pool:
+        together = list(pool.map(go, texts))
+    for a, b in zip(alone, together):
+        assert len(a) == len(b) and all(np.array_equal(x, y) for x, y in zip(a, b))
 
 
 CHILD = """
