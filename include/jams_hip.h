@@ -227,7 +227,7 @@ int jh_set_replicas(jh_ctx *ctx, int nrep, const int64_t *offsets, const double 
 int jh_reduce_magnetisation_replicas(jh_ctx *ctx, double *out);
 
 /* ---- launch shape -------------------------------------------------------- */
-/* Run jh_step as replays of one captured hipGraph of `steps` Heun steps
+/* Run jh_step as replays of one hipGraph of `steps` Heun steps
  * (whatever is left over runs as plain launches); 0 disables graphs.  Without
  * a call, contexts of up to 2^18 spins replay a 20-step graph of their own
  * once they have run 500 steps, with the same results, and plain launches

@@ -5,7 +5,7 @@ Each replica is a JAMS config set up by the C++ host layer without a device
 noise seed and applied field.  The batch concatenates the replicas into one
 engine context in which replica r owns the spins [offsets[r], offsets[r+1])
 (jh_set_replicas): one launch per Heun phase covers every replica, the step
-loop can replay a captured hipGraph (jh_set_graph_steps), and the exchange
+loop can replay a hipGraph (jh_set_graph_steps), and the exchange
 format and workgroup size are picked by timing (jh_autotune).  A replica
 evolves bit for bit as it would in a context of its own.
 """

@@ -41,6 +41,7 @@
 #include "jh_device.h"
 #include "jh_dipole.h"
 #include "jh_fft.h"
+#include "jh_graph.h"
 
 namespace jh {
 
@@ -663,14 +664,14 @@ hipError_t run_direct_z(const Pass<T> &p, bool inverse, hipStream_t st) {
   const unsigned blocks = (unsigned)((p.nlines + t - 1) / t);
   const int lmax = std::max(inverse ? p.n_out : p.n_in, (p.n + 1) / 2);
   if (lmax <= 8) {
-    if (inverse) hipLaunchKernelGGL((k_dip_z_direct_inv<T, 8>), dim3(blocks), dim3(t), lds, st, p);
-    else hipLaunchKernelGGL((k_dip_z_direct_fwd<T, 8>), dim3(blocks), dim3(t), lds, st, p);
+    if (inverse) enqueue((k_dip_z_direct_inv<T, 8>), dim3(blocks), dim3(t), lds, st, p);
+    else enqueue((k_dip_z_direct_fwd<T, 8>), dim3(blocks), dim3(t), lds, st, p);
   } else if (lmax <= 16) {
-    if (inverse) hipLaunchKernelGGL((k_dip_z_direct_inv<T, 16>), dim3(blocks), dim3(t), lds, st, p);
-    else hipLaunchKernelGGL((k_dip_z_direct_fwd<T, 16>), dim3(blocks), dim3(t), lds, st, p);
+    if (inverse) enqueue((k_dip_z_direct_inv<T, 16>), dim3(blocks), dim3(t), lds, st, p);
+    else enqueue((k_dip_z_direct_fwd<T, 16>), dim3(blocks), dim3(t), lds, st, p);
   } else {
-    if (inverse) hipLaunchKernelGGL((k_dip_z_direct_inv<T, 32>), dim3(blocks), dim3(t), lds, st, p);
-    else hipLaunchKernelGGL((k_dip_z_direct_fwd<T, 32>), dim3(blocks), dim3(t), lds, st, p);
+    if (inverse) enqueue((k_dip_z_direct_inv<T, 32>), dim3(blocks), dim3(t), lds, st, p);
+    else enqueue((k_dip_z_direct_fwd<T, 32>), dim3(blocks), dim3(t), lds, st, p);
   }
   return hipGetLastError();
 }
@@ -968,11 +969,11 @@ hipError_t run_pass(Pass<T> p, hipStream_t st) {
     if (e != hipSuccess) return e;
   }
   if (p.inverse)
-    hipLaunchKernelGGL((fft::k_fft_pass<T, LD, ST, true>), dim3((unsigned)blocks),
-                       dim3(fft::kThreads), lds, st, p);
+    enqueue((fft::k_fft_pass<T, LD, ST, true>), dim3((unsigned)blocks),
+            dim3(fft::kThreads), lds, st, p);
   else
-    hipLaunchKernelGGL((fft::k_fft_pass<T, LD, ST, false>), dim3((unsigned)blocks),
-                       dim3(fft::kThreads), lds, st, p);
+    enqueue((fft::k_fft_pass<T, LD, ST, false>), dim3((unsigned)blocks),
+            dim3(fft::kThreads), lds, st, p);
   return hipGetLastError();
 }
 
@@ -985,9 +986,9 @@ hipError_t launch_zy_inv(const ZYFused<T> &q, int lwk, unsigned blocks, int nt, 
                               : reinterpret_cast<const void *>(&k_dip_zy_inv<T, LM, 0>);
   if (lds > 64 * 1024)
     DCHK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-  if (lwk == 3) hipLaunchKernelGGL((k_dip_zy_inv<T, LM, 3>), dim3(blocks), dim3(nt), lds, st, q);
-  else if (lwk == 5) hipLaunchKernelGGL((k_dip_zy_inv<T, LM, 5>), dim3(blocks), dim3(nt), lds, st, q);
-  else hipLaunchKernelGGL((k_dip_zy_inv<T, LM, 0>), dim3(blocks), dim3(nt), lds, st, q);
+  if (lwk == 3) enqueue((k_dip_zy_inv<T, LM, 3>), dim3(blocks), dim3(nt), lds, st, q);
+  else if (lwk == 5) enqueue((k_dip_zy_inv<T, LM, 5>), dim3(blocks), dim3(nt), lds, st, q);
+  else enqueue((k_dip_zy_inv<T, LM, 0>), dim3(blocks), dim3(nt), lds, st, q);
   return hipGetLastError();
 }
 
@@ -1115,9 +1116,9 @@ class DipoleFFTImpl : public DipoleFFT {
     const size_t lds = ((size_t)q.n * q.lw + (x_lwk(q.lw) ? kTw512 : q.n)) * sizeof(T2);
     const unsigned blocks = (unsigned)(Q2 * q.nyb);
     if (x_lwk(q.lw) == 6)
-      hipLaunchKernelGGL((k_dip_x_fused<T, 6>), dim3(blocks), dim3(xf_threads<T>(q.by)), lds, st, q);
+      enqueue((k_dip_x_fused<T, 6>), dim3(blocks), dim3(xf_threads<T>(q.by)), lds, st, q);
     else
-      hipLaunchKernelGGL((k_dip_x_fused<T, 0>), dim3(blocks), dim3(xf_threads<T>(q.by)), lds, st, q);
+      enqueue((k_dip_x_fused<T, 0>), dim3(blocks), dim3(xf_threads<T>(q.by)), lds, st, q);
     return hipGetLastError();
   }
 
@@ -1139,9 +1140,9 @@ class DipoleFFTImpl : public DipoleFFT {
       DCHK(pl.Wc.alloc((size_t)ncomp * M));
     }
     const int64_t blocks = ((int64_t)ncomp * M + 255) / 256;
-    hipLaunchKernelGGL((k_dip_extract<T>), dim3((unsigned)blocks), dim3(256), 0, st,
-                       (const double2 *)Fsetup.p, (int64_t)P[2], Q2, (int64_t)P[0] * P[1], ncomp,
-                       real_tensor, pl.Wr.p, pl.Wc.p);
+    enqueue((k_dip_extract<T>), dim3((unsigned)blocks), dim3(256), 0, st,
+            (const double2 *)Fsetup.p, (int64_t)P[2], Q2, (int64_t)P[0] * P[1], ncomp,
+            real_tensor, pl.Wr.p, pl.Wc.p);
     DCHK(hipGetLastError());
     DCHK(hipStreamSynchronize(st));
     const int by = fused_lines<T>();
@@ -1151,8 +1152,8 @@ class DipoleFFTImpl : public DipoleFFT {
       const int nyb = (P[1] + by - 1) / by;
       const int64_t total = Q2 * nyb * 6 * (int64_t)P[0] * by;
       DCHK(pl.Wf.alloc((size_t)total));
-      hipLaunchKernelGGL((k_dip_w_fused<T>), dim3((unsigned)((total + 255) / 256)), dim3(256), 0,
-                         st, (const T *)pl.Wr.p, pl.Wf.p, M, P[0], P[1], lby, nyb, total);
+      enqueue((k_dip_w_fused<T>), dim3((unsigned)((total + 255) / 256)), dim3(256), 0,
+              st, (const T *)pl.Wr.p, pl.Wf.p, M, P[0], P[1], lby, nyb, total);
       DCHK(hipGetLastError());
       DCHK(hipStreamSynchronize(st));
       pl.Wr.release();
@@ -1319,14 +1320,14 @@ class DipoleFFTImpl : public DipoleFFT {
     const size_t lds = zy_lds<T>(q.lw);
     const bool k3 = zy_fwd_lwk(q.lw) == 3;
     if (L[2] <= 8) {
-      if (k3) hipLaunchKernelGGL((k_dip_zy_fwd<T, 8, 3>), dim3(blocks), dim3(nt), lds, st, q);
-      else hipLaunchKernelGGL((k_dip_zy_fwd<T, 8, 0>), dim3(blocks), dim3(nt), lds, st, q);
+      if (k3) enqueue((k_dip_zy_fwd<T, 8, 3>), dim3(blocks), dim3(nt), lds, st, q);
+      else enqueue((k_dip_zy_fwd<T, 8, 0>), dim3(blocks), dim3(nt), lds, st, q);
     } else if (L[2] <= 16) {
-      if (k3) hipLaunchKernelGGL((k_dip_zy_fwd<T, 16, 3>), dim3(blocks), dim3(nt), lds, st, q);
-      else hipLaunchKernelGGL((k_dip_zy_fwd<T, 16, 0>), dim3(blocks), dim3(nt), lds, st, q);
+      if (k3) enqueue((k_dip_zy_fwd<T, 16, 3>), dim3(blocks), dim3(nt), lds, st, q);
+      else enqueue((k_dip_zy_fwd<T, 16, 0>), dim3(blocks), dim3(nt), lds, st, q);
     } else {
-      if (k3) hipLaunchKernelGGL((k_dip_zy_fwd<T, 32, 3>), dim3(blocks), dim3(nt), lds, st, q);
-      else hipLaunchKernelGGL((k_dip_zy_fwd<T, 32, 0>), dim3(blocks), dim3(nt), lds, st, q);
+      if (k3) enqueue((k_dip_zy_fwd<T, 32, 3>), dim3(blocks), dim3(nt), lds, st, q);
+      else enqueue((k_dip_zy_fwd<T, 32, 0>), dim3(blocks), dim3(nt), lds, st, q);
     }
     return hipGetLastError();
   }
@@ -1387,11 +1388,11 @@ class DipoleFFTImpl : public DipoleFFT {
       {
         const int64_t blocks = (M + 255) / 256;
         if (real_tensor)
-          hipLaunchKernelGGL((k_dip_mult_real<T>), dim3((unsigned)blocks), dim3(256), 0, st, pl.K.p,
-                             (const T *)pl.Wr.p, M);
+          enqueue((k_dip_mult_real<T>), dim3((unsigned)blocks), dim3(256), 0, st, pl.K.p,
+                  (const T *)pl.Wr.p, M);
         else
-          hipLaunchKernelGGL((k_dip_mult_cplx<T>), dim3((unsigned)blocks), dim3(256), 0, st, pl.K.p,
-                             (const T2 *)pl.Wc.p, M, nb);
+          enqueue((k_dip_mult_cplx<T>), dim3((unsigned)blocks), dim3(256), 0, st, pl.K.p,
+                  (const T2 *)pl.Wc.p, M, nb);
         DCHK(hipGetLastError());
       }
       // x inverse, outputs x < L0

@@ -84,7 +84,7 @@ constexpr int64_t kLnAutoMinRow = 24;           // neighbours per row from which
 // typically about a second, against a phase of under a millisecond for a few
 // million spins
 constexpr unsigned kStepPollLimit = 1u << 20;
-// Small contexts replay a captured graph of kAutoGraphSteps steps by
+// Small contexts replay a graph of kAutoGraphSteps steps by
 // themselves, once they have run kAutoGraphAfter steps since they were laid
 // out: a launch in a graph costs the GPU about 0.8 us less than a plain one (sc
 // 16^3 thermal 11.9 -> 10.1 us per step, bcc 32^3 x 2 14.0 -> 12.3; bcc 64^3 x 2
@@ -377,7 +377,7 @@ struct jh_ctx {
   int step_launch = JH_STEP_LAUNCH_TWO;
   DevBuf<unsigned> step_sync;
   int cus = 0;
-  int graph_steps = 0;              // steps per captured graph (0: plain launches,
+  int graph_steps = 0;              // steps per graph (0: plain launches,
                                     // or the engine's own choice, auto_graph)
   bool auto_graph = true;
   int64_t steps_run = 0;            // plain steps since the launches last changed
@@ -1832,7 +1832,7 @@ const char *persistent_unfit(const jh_ctx *c) {
 }
 
 // The grid barrier's words, zero before the first persistent launch (set up
-// outside any captured graph: prepare runs before a capture)
+// not in a graph: prepare runs before one is built)
 void ensure_step_sync(jh_ctx *c) {
   if (c->step_sync.p) return;
   c->step_sync.alloc(4);
@@ -2084,8 +2084,8 @@ void enqueue_step(jh_ctx *c, KParams p) {
   launch_phase(c, p, 1);
 }
 
-// Capture `steps` steps.  Their kernels read the step counter as
-// *c->dstep + k (k, the step's place in the graph, is baked into its
+// The launches of `steps` steps as a graph.  Their kernels read the step
+// counter as *c->dstep + k (k, the step's place in the graph, is baked into its
 // parameters), and the host sets *c->dstep once per replay with a one-thread
 // kernel outside the graph (no memset nodes).
 void build_graph(jh_ctx *c, int steps) {
@@ -2093,19 +2093,21 @@ void build_graph(jh_ctx *c, int steps) {
   if (!c->dstep.p) c->dstep.alloc(1);
   KParams p = make_params(c);
   p.dstep = c->dstep.p;
-  HIPCHK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
+  HIPCHK(hipGraphCreate(&c->graph, 0));
+  GraphChain chain{c->graph};
+  graph_chain = &chain;
   try {
     for (int k = 0; k < steps; ++k) {
       p.step = (uint64_t)k;
       enqueue_step(c, p);
     }
   } catch (...) {
-    hipGraph_t g = nullptr;
-    (void)hipStreamEndCapture(c->stream, &g);
-    if (g) (void)hipGraphDestroy(g);
+    graph_chain = nullptr;
+    c->drop_graph();
     throw;
   }
-  HIPCHK(hipStreamEndCapture(c->stream, &c->graph));
+  graph_chain = nullptr;
+  HIPCHK(chain.err);
   HIPCHK(hipGraphInstantiate(&c->gexec, c->graph, nullptr, nullptr, 0));
 }
 

@@ -1956,17 +1956,17 @@ static hipError_t launch_heun_t(const KParams &p, int phase, int bs, hipStream_t
   // class table, CM_ONE without); the GEN forms per lane
   const bool uc = p.cls != nullptr;
   if (phase == 0 && !gen && uc)
-    hipLaunchKernelGGL((k_heun<PREC, XVk, 0, false, CM_SPLIT>), dim3((unsigned)nb), dim3(bs), lds, st, p);
+    enqueue((k_heun<PREC, XVk, 0, false, CM_SPLIT>), dim3((unsigned)nb), dim3(bs), lds, st, p);
   else if (phase == 0 && !gen)
-    hipLaunchKernelGGL((k_heun<PREC, XVk, 0, false, CM_ONE>), dim3((unsigned)nb), dim3(bs), lds, st, p);
+    enqueue((k_heun<PREC, XVk, 0, false, CM_ONE>), dim3((unsigned)nb), dim3(bs), lds, st, p);
   else if (phase == 0)
-    hipLaunchKernelGGL((k_heun<PREC, XVk, 0, true, CM_LANE>), dim3((unsigned)nb), dim3(bs), lds, st, p);
+    enqueue((k_heun<PREC, XVk, 0, true, CM_LANE>), dim3((unsigned)nb), dim3(bs), lds, st, p);
   else if (!gen && uc)
-    hipLaunchKernelGGL((k_heun<PREC, XVk, 1, false, CM_SPLIT>), dim3((unsigned)nb), dim3(bs), lds, st, p);
+    enqueue((k_heun<PREC, XVk, 1, false, CM_SPLIT>), dim3((unsigned)nb), dim3(bs), lds, st, p);
   else if (!gen)
-    hipLaunchKernelGGL((k_heun<PREC, XVk, 1, false, CM_ONE>), dim3((unsigned)nb), dim3(bs), lds, st, p);
+    enqueue((k_heun<PREC, XVk, 1, false, CM_ONE>), dim3((unsigned)nb), dim3(bs), lds, st, p);
   else
-    hipLaunchKernelGGL((k_heun<PREC, XVk, 1, true, CM_LANE>), dim3((unsigned)nb), dim3(bs), lds, st, p);
+    enqueue((k_heun<PREC, XVk, 1, true, CM_LANE>), dim3((unsigned)nb), dim3(bs), lds, st, p);
   return hipGetLastError();
 }
 
@@ -2029,7 +2029,7 @@ static hipError_t launch_heun_step_k(const KParams &p, int bs, int cus, unsigned
   KParams q = p;
   q.g32 = p.w32;
   q.w32 = const_cast<float *>(p.g32);
-  hipLaunchKernelGGL(fn, dim3((unsigned)g), dim3(bs), lds, st, p, q, sync, limit);
+  enqueue(fn, dim3((unsigned)g), dim3(bs), lds, st, p, q, sync, limit);
   return hipGetLastError();
 }
 
@@ -2094,7 +2094,7 @@ static hipError_t launch_heun_many_t(const KParams &p, int nsteps, hipStream_t s
                                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
   }
-  hipLaunchKernelGGL(fn, dim3(1), dim3(threads), lds, st, p, nsteps, off);
+  enqueue(fn, dim3(1), dim3(threads), lds, st, p, nsteps, off);
   return hipGetLastError();
 }
 
@@ -2141,7 +2141,7 @@ static hipError_t launch_heun_st_k(const KParams &p, const StView &v, size_t lds
     if (e != hipSuccess) return e;
   }
   const int64_t nwg = (int64_t)v.nb * v.nbx * v.nby * v.nbz;
-  hipLaunchKernelGGL(fn, dim3((unsigned)nwg), dim3(64 * v.wx * v.wy), lds, st, p, v);
+  enqueue(fn, dim3((unsigned)nwg), dim3(64 * v.wx * v.wy), lds, st, p, v);
   return hipGetLastError();
 }
 
@@ -2177,13 +2177,13 @@ static hipError_t launch_heun_ln_t(const KParams &p, const LnView &v, int phase,
   const bool gen = p.has_ac || p.ani_power != 2;
   const bool one = p.cls == nullptr;
   if (phase == 0) {
-    if (gen) hipLaunchKernelGGL((k_heun_ln<PREC, DIAG, 0, true, P, false>), grid, block, lds, st, p, v);
-    else if (one) hipLaunchKernelGGL((k_heun_ln<PREC, DIAG, 0, false, P, true>), grid, block, lds, st, p, v);
-    else hipLaunchKernelGGL((k_heun_ln<PREC, DIAG, 0, false, P, false>), grid, block, lds, st, p, v);
+    if (gen) enqueue((k_heun_ln<PREC, DIAG, 0, true, P, false>), grid, block, lds, st, p, v);
+    else if (one) enqueue((k_heun_ln<PREC, DIAG, 0, false, P, true>), grid, block, lds, st, p, v);
+    else enqueue((k_heun_ln<PREC, DIAG, 0, false, P, false>), grid, block, lds, st, p, v);
   } else {
-    if (gen) hipLaunchKernelGGL((k_heun_ln<PREC, DIAG, 1, true, P, false>), grid, block, lds, st, p, v);
-    else if (one) hipLaunchKernelGGL((k_heun_ln<PREC, DIAG, 1, false, P, true>), grid, block, lds, st, p, v);
-    else hipLaunchKernelGGL((k_heun_ln<PREC, DIAG, 1, false, P, false>), grid, block, lds, st, p, v);
+    if (gen) enqueue((k_heun_ln<PREC, DIAG, 1, true, P, false>), grid, block, lds, st, p, v);
+    else if (one) enqueue((k_heun_ln<PREC, DIAG, 1, false, P, true>), grid, block, lds, st, p, v);
+    else enqueue((k_heun_ln<PREC, DIAG, 1, false, P, false>), grid, block, lds, st, p, v);
   }
   return hipGetLastError();
 }
@@ -2217,11 +2217,11 @@ static hipError_t launch_rk4_t(const KParams &p, int bs, hipStream_t st) {
   const int64_t nb = (p.n + bs - 1) / bs;
   const size_t lds = table_lds(p, PREC, XVk);
   if (p.has_ac || p.ani_power != 2)
-    hipLaunchKernelGGL((k_rk4<PREC, XVk, true, false>), dim3((unsigned)nb), dim3(bs), lds, st, p);
+    enqueue((k_rk4<PREC, XVk, true, false>), dim3((unsigned)nb), dim3(bs), lds, st, p);
   else if (p.cls)
-    hipLaunchKernelGGL((k_rk4<PREC, XVk, false, false>), dim3((unsigned)nb), dim3(bs), lds, st, p);
+    enqueue((k_rk4<PREC, XVk, false, false>), dim3((unsigned)nb), dim3(bs), lds, st, p);
   else
-    hipLaunchKernelGGL((k_rk4<PREC, XVk, false, true>), dim3((unsigned)nb), dim3(bs), lds, st, p);
+    enqueue((k_rk4<PREC, XVk, false, true>), dim3((unsigned)nb), dim3(bs), lds, st, p);
   return hipGetLastError();
 }
 
@@ -2262,12 +2262,12 @@ hipError_t launch_rk4(const KParams &p, int prec, int xv, int bs, hipStream_t st
 
 hipError_t launch_reduce_replicas(const KParams &p, const int64_t *off, int nrep, double *out,
                                   hipStream_t st) {
-  hipLaunchKernelGGL(k_reduce_replicas, dim3((unsigned)nrep), dim3(kBlock), 0, st, p, off, out);
+  enqueue(k_reduce_replicas, dim3((unsigned)nrep), dim3(kBlock), 0, st, p, off, out);
   return hipGetLastError();
 }
 
 hipError_t launch_set_step(uint64_t *step, uint64_t value, hipStream_t st) {
-  hipLaunchKernelGGL(k_set_step, dim3(1), dim3(64), 0, st, step, value);
+  enqueue(k_set_step, dim3(1), dim3(64), 0, st, step, value);
   return hipGetLastError();
 }
 
@@ -2275,7 +2275,7 @@ template <int PREC, int XVk>
 static hipError_t launch_field_t(const KParams &p, int term, double *out, hipStream_t st) {
   const int64_t nb = (p.n + kBlock - 1) / kBlock;
   const size_t lds = table_lds(p, PREC, XVk);
-  hipLaunchKernelGGL((k_field<PREC, XVk>), dim3((unsigned)nb), dim3(kBlock), lds, st, p, term, out);
+  enqueue((k_field<PREC, XVk>), dim3((unsigned)nb), dim3(kBlock), lds, st, p, term, out);
   return hipGetLastError();
 }
 
@@ -2318,27 +2318,27 @@ hipError_t launch_vec_layout(const double *in, double *out, int64_t n, int order
   const auto fn = spin ? (to_host ? k_vec_layout<true, true> : k_vec_layout<true, false>)
                        : (to_host ? k_vec_layout<false, true> : k_vec_layout<false, false>);
   const int64_t nb = (n + kBlock - 1) / kBlock;
-  hipLaunchKernelGGL(fn, dim3((unsigned)nb), dim3(kBlock), 0, st, in, out, n, order_nb, order_cells);
+  enqueue(fn, dim3((unsigned)nb), dim3(kBlock), 0, st, in, out, n, order_nb, order_cells);
   return hipGetLastError();
 }
 
 hipError_t launch_noise(const KParams &p, double *out, hipStream_t st) {
   const int64_t nb = (p.n + kBlock - 1) / kBlock;
-  hipLaunchKernelGGL(k_noise, dim3((unsigned)nb), dim3(kBlock), 0, st, p, out);
+  enqueue(k_noise, dim3((unsigned)nb), dim3(kBlock), 0, st, p, out);
   return hipGetLastError();
 }
 
 hipError_t launch_to_f32(const double *a, float *b, int64_t n, hipStream_t st) {
   const int64_t nb = (n + kBlock - 1) / kBlock;
-  hipLaunchKernelGGL(k_to_f32, dim3((unsigned)nb), dim3(kBlock), 0, st, a, b, n);
+  enqueue(k_to_f32, dim3((unsigned)nb), dim3(kBlock), 0, st, a, b, n);
   return hipGetLastError();
 }
 
 hipError_t launch_reduce(const KParams &p, int mode, const double *h, double *partial,
                          double *out, hipStream_t st) {
   const int64_t nb = (p.n + kBlock - 1) / kBlock;
-  hipLaunchKernelGGL(k_reduce, dim3((unsigned)nb), dim3(kBlock), 0, st, p, mode, h, partial);
-  hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(kBlock), 0, st, (const double *)partial, nb, out);
+  enqueue(k_reduce, dim3((unsigned)nb), dim3(kBlock), 0, st, p, mode, h, partial);
+  enqueue(k_reduce_final, dim3(1), dim3(kBlock), 0, st, (const double *)partial, nb, out);
   return hipGetLastError();
 }
 

@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include "jh_graph.h"
 #include "jh_internal.h"
 
 namespace jh {

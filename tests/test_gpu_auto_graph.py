@@ -1,8 +1,10 @@
-"""Small contexts replay a captured graph of their own accord after enough
+"""Small contexts replay a graph of their own accord after enough
 plain steps: the same bits as calls too short for a replay, replay after
 replay, with reductions, field evaluations and set-up changes in between."""
+import ctypes
 import subprocess
 import sys
+import threading
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
@@ -105,7 +107,7 @@ def test_noise_set_before_every_few_steps(chosen):
 
 
 def test_contexts_on_several_threads():
-    """Each thread sets contexts up, steps them past the point where they capture
+    """Each thread sets contexts up, steps them past the point where they build
     a graph and reads them, while the others do the same: the bits of the same
     runs one after the other."""
     texts = [configs.sc_config(L=(13, 11, 12), temperature=20.0, seed=3),
@@ -114,7 +116,7 @@ def test_contexts_on_several_threads():
 
     def go(text):
         out = []
-        for _ in range(3):
+        for _ in range(6):
             s = Simulation(text, device=0, output_dir="/tmp")
             e = s.engine()
             for n in (490, 30, 75):
@@ -132,6 +134,35 @@ def test_contexts_on_several_threads():
         together = list(pool.map(go, texts))
     for a, b in zip(alone, together):
         assert len(a) == len(b) and all(np.array_equal(x, y) for x, y in zip(a, b))
+
+
+def test_building_a_graph_leaves_other_threads_alone():
+    """Copies on the legacy stream by another thread of the process, which a
+    stream capture anywhere in it would have the runtime refuse."""
+    sim = Simulation(CASES["heun"], device=0, output_dir="/tmp")
+    e = sim.engine()
+    hip = e.lib  # the engine's own HIP library is found through it
+    dev, host = ctypes.c_void_p(), (ctypes.c_char * 64)()
+    assert hip.hipMalloc(ctypes.byref(dev), ctypes.c_size_t(64)) == 0
+    done, results = threading.Event(), []
+
+    def copy():
+        while not done.is_set():
+            results.append(hip.hipMemcpy(dev, host, ctypes.c_size_t(64), 1))
+
+    t = threading.Thread(target=copy)
+    t.start()
+    try:
+        for k in range(20):
+            e.set_graph_steps(300 + k)
+            e.step(300 + k)
+    finally:
+        done.set()
+        t.join()
+    e.synchronize()
+    assert hip.hipFree(dev) == 0
+    assert len(results) > 20 and not any(results)
+    sim.close()
 
 
 CHILD = """
